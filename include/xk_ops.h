@@ -346,7 +346,10 @@ int xk_gdn_conv_gating_decode(
  *   first.  K = 128, V a multiple of 32.  q, k, v 16-byte aligned, o
  *   8-byte aligned (else XK_ERR_INVALID).
  *   workspace >= xk_gdn_chunk_workspace_bytes(total_tokens, N, HV) bytes,
- *   256-byte aligned (chunk offsets + per-chunk inverse blocks).
+ *   256-byte aligned (chunk offsets + per-chunk inverse blocks).  For batches
+ *   that leave most compute units idle behind long sequences the size
+ *   includes room to run segments of them in parallel; a workspace that holds
+ *   the rest but not that is accepted and runs every sequence in order.
  */
 int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                      int64_t HV);
@@ -364,9 +367,8 @@ int xk_gdn_chunk_fwd(
  * harnesses that forbid hipMalloc).  No counterpart in the reference.
  * Same arguments and results as xk_gdn_chunk_fwd (the same kernels run);
  * the workspace is a static device buffer of 64 MiB that the library holds
- * on every GPU it runs on until the process ends.  Calls whose
- * xk_gdn_chunk_workspace_bytes(total_tokens, N, HV) exceeds 64 MiB return
- * XK_ERR_SCRATCH (e.g. up to ~6,700 tokens at HV = 32, ~27,000 at HV = 8).
+ * on every GPU it runs on until the process ends.  Calls whose workspace
+ * without room for segments exceeds 64 MiB return XK_ERR_SCRATCH (e.g. up to ~6,700 tokens at HV = 32, ~27,000 at HV = 8).
  * The call allocates nothing; `stream` must belong to the current device.
  * Every call on one GPU shares that GPU's buffer: calls that overlap in
  * time on one GPU (other streams, other host threads) race.

@@ -1,0 +1,127 @@
+"""Chunked gated delta rule on batches whose sequences are cut into segments
+that run in parallel (few heads, long sequences), against the oracle and
+against the same call in a workspace one byte too small for the segments,
+which runs whole sequences in order.
+
+The two paths differ only in how the state reaches a segment: its entry state
+passes through the segments' transition matrices, whose products keep ~16
+mantissa bits like every state product of a chunk.  Each of the two paths is
+within 3.1e-5 (RMS + |value|) of the fp32 reference over the chunked tests
+(errors of 2^-17 of the state's size per product, over the few chunks for
+which the delta rule remembers them), so they may differ by twice that:
+6.2e-5 of the RMS and of the value.
+Outputs are sums of products of operands rounded to bf16 (the state's hi part,
+v_new); a difference that small can flip the last bit of one operand, which
+moves an output by up to 2^-8 of one term of its sum, a term being at most of
+the outputs' own size: 2^-7 of their RMS beside one bf16 step (2^-7 of the
+value) of the output itself are allowed."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from oracle import gdn as og
+from state_tol import assert_state_close
+
+pytestmark = pytest.mark.gpu
+
+O_TOL = dict(rtol=1.6e-2, atol=1e-2)
+
+
+def _inputs(lens, H, HV, seed=0, V=128):
+    gen = torch.Generator().manual_seed(seed)
+    T = sum(lens)
+    q = torch.randn(1, T, H, 128, generator=gen).bfloat16()
+    k = torch.randn(1, T, H, 128, generator=gen).bfloat16()
+    v = torch.randn(1, T, HV, V, generator=gen).bfloat16()
+    # Some heads forget within a chunk, some keep their state throughout.
+    g = -F.softplus(torch.randn(1, T, HV, generator=gen)) * torch.logspace(-4, 0, HV)
+    beta = torch.sigmoid(torch.randn(1, T, HV, generator=gen)).bfloat16()
+    h0 = torch.randn(len(lens), HV, 128, V, generator=gen)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    return q, k, v, g, beta, h0, cu
+
+
+def _run(dev, q, k, v, g, beta, h0, cu, segments=True, l2norm=True, bufs=None):
+    from torch_npu_ops_amd import _lib, ops
+    _, T, H, K = q.shape
+    HV, V, N = v.shape[2], v.shape[3], cu.numel() - 1
+    need = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV)
+    t = [x.to(dev).contiguous() for x in (q, k, v, g.float(), beta, h0, cu)] if bufs is None else bufs
+    o = torch.empty(1, T, HV, V, dtype=torch.bfloat16, device=dev)
+    fin = torch.empty(N, HV, K, V, device=dev)
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
+
+    def call():
+        st = _lib.lib().xk_gdn_chunk_fwd(
+            t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), _lib.XK_BF16, t[3].data_ptr(),
+            _lib.XK_F32, t[4].data_ptr(), _lib.XK_BF16, o.data_ptr(), t[5].data_ptr(),
+            fin.data_ptr(), t[6].data_ptr(), _lib.XK_I32, N, T, H, HV, K, V, K ** -0.5,
+            int(l2norm), ws.data_ptr(), need if segments else need - 1, ops._stream(o))
+        _lib.check(st, "xk_gdn_chunk_fwd")
+    call()
+    torch.cuda.synchronize()
+    return o, fin, call
+
+
+def _same(a, b):
+    (o1, f1, _), (o2, f2, _) = a, b
+    o1, o2 = o1.float(), o2.float()
+    rms = o2[o2.isfinite()].pow(2).mean().sqrt().item()
+    torch.testing.assert_close(o1, o2, rtol=2 ** -7, atol=2 ** -7 * rms, equal_nan=True)
+    rms = f2[f2.isfinite()].pow(2).mean().sqrt().item()
+    torch.testing.assert_close(f1, f2, rtol=6.2e-5, atol=6.2e-5 * rms, equal_nan=True)
+
+
+# One sequence at its shortest segmented length, odd lengths around chunk and
+# segment edges, many segments; ragged batches with empty and one-token
+# sequences; one and three 64-column tiles.
+@pytest.mark.parametrize("lens,H,HV,V", [
+    ([1024], 4, 8, 128), ([1025], 2, 4, 128), ([2111], 1, 2, 128), ([4095], 2, 2, 128),
+    ([9000], 1, 2, 128), ([2500], 2, 6, 64), ([64 * 31 + 1, 0, 1, 700], 2, 4, 128),
+    ([3000, 200, 1500], 1, 1, 128)])
+def test_segments(dev, lens, H, HV, V):
+    x = _inputs(lens, H, HV, seed=sum(lens), V=V)
+    out = _run(dev, *x)
+    _same(out, _run(dev, *x, segments=False))
+    q, k, v, g, beta, h0, cu = x
+    ro, rs = og.chunk_gdn(q, k, v, g, beta, None, h0, cu, use_qk_l2norm=True)
+    torch.testing.assert_close(out[0].float().cpu(), ro, **O_TOL)
+    assert_state_close(out[1].cpu(), rs)
+
+
+def test_segments_in_a_graph(dev):
+    x = _inputs([3001], 2, 4, seed=3)
+    o, fin, call = _run(dev, *x)
+    want = o.clone(), fin.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        o.zero_()
+        fin.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want[0]) and torch.equal(fin, want[1])
+
+
+def test_growing_transition_runs_in_order(dev):
+    """Keys of norm > 1 along one direction: 1 - beta |k|^2 < -1, so the
+    transition grows without bound and the head must run in order, bit for
+    bit as without segments; the other head stays segmented."""
+    q, k, v, g, beta, h0, cu = _inputs([2048], 2, 2, seed=5)
+    k = F.normalize(k.float(), dim=-1)
+    k[:, :, 0] = F.normalize(k[0, 0, 0], dim=-1) * 1.425  # |k|^2 = 2.03
+    x = (q, k.bfloat16(), v, g, beta.masked_fill(torch.arange(2) == 0, 1.0), h0, cu)
+    x[3][..., 0] = 0.0
+    a, b = _run(dev, *x, l2norm=False), _run(dev, *x, segments=False, l2norm=False)
+    assert torch.equal(a[0][:, :, 0], b[0][:, :, 0]) and torch.equal(a[1][:, 0], b[1][:, 0])
+    _same((a[0][:, :, 1:], a[1][:, 1:], None), (b[0][:, :, 1:], b[1][:, 1:], None))
+
+
+def test_nan_value_spreads_no_further(dev):
+    """A NaN value reaches the same outputs as in order, and no transition."""
+    q, k, v, g, beta, h0, cu = _inputs([3000], 1, 2, seed=7)
+    v[0, 1500, 1, 17] = float("nan")
+    a, b = _run(dev, q, k, v, g, beta, h0, cu), _run(dev, q, k, v, g, beta, h0, cu, segments=False)
+    assert b[1][:, 1, :, 17].isnan().all() and not b[1][:, 1, :, 64:].isnan().any()
+    _same(a, b)

@@ -16,8 +16,9 @@
 // (npu_l2norm_last_dim, x / sqrt(sum x^2 + 1e-6)) is folded in as per-token
 // row scales, so the matrix products always see the exact bf16 inputs.
 //
-// Three launches, no host synchronisation (capturable in a hipGraph):
-//  * P0 (one small block) turns cu_seqlens into chunk offsets.
+// Two to five launches, no host synchronisation (capturable in a hipGraph):
+//  * P0 (one small block, above 64 sequences) turns cu_seqlens into chunk
+//    offsets.
 //  * P1, fully parallel, one wave per (chunk, v-head), computes everything
 //    that does not depend on the carried state and writes one record per
 //    (chunk, head) to the workspace:
@@ -40,6 +41,9 @@
 //    and emits o = cq (Q S) + Aq Vn.  Every global operand of chunk c+1 is
 //    loaded while chunk c computes.  Blocks of one (sequence, head) share an
 //    XCD (block id mod 8) and thus its L2 for the shared q/k/record reads.
+//    Where few blocks would leave the chip idle behind long sequences, P2
+//    runs as three passes over segments of them ("Segments" below).
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -96,10 +100,108 @@ struct ChunkParams {
   int H, HV;
   float scale;
   int l2norm;
+  // Segmented state pass (below); seg_max 0: whole sequences only.
+  int seg_max;        // segments the workspace holds
+  int seg_cus, seg_nvt;  // compute units and V tiles the plan counts on
+  int32_t* seg_len;   // the plan: chunks per segment
+  char* seg_m;        // [seg_max, HV]: transition of a segment, kSegImg bytes of operand images
+  float* seg_b;       // [seg_max, HV, K, V]: its end state from zero (the first one's: from h0),
+                      // then the state after it
+  int32_t* seg_over;  // [seg_max, HV, 2]: a transition entry of that half exceeds kSegLimit
+  int32_t* seg_bad;   // [N, HV]: the head runs in order
 };
 
 __device__ __forceinline__ char* rec_at(const ChunkParams& p, int64_t c, int hv) {
   return p.rec + (c * p.HV + hv) * static_cast<int64_t>(kRec);
+}
+
+// ---------------------------------------------------------------------------
+// Segments.  A sequence's chunk chain is serial, so few (sequence, head, V
+// tile) blocks leave most CUs idle behind a long chain.  A sequence may be
+// cut into segments of `len` chunks that run in parallel:
+//  * kSegSum: per segment, the state after it from a zero state (B; the
+//    first segment starts from the initial state instead) and its transition
+//    M (the same recurrence without values, from the identity: K more
+//    columns), without outputs;
+//  * gdn_chunk_combine_kernel: the states at the segment boundaries,
+//    S <- M_i S + B_i in order;
+//  * kSegOut: every segment from its entry state, with outputs.
+// The work of the state pass grows about 2.4 times, so this pays only where
+// the chip is idle.  len is chosen on the device, where the lengths are
+// known: one block of the prep kernel evaluates seg_cost for 1 .. 64
+// segments of the longest sequence, one candidate per lane.  The host
+// launches these passes if a batch of this size can gain (seg_plan).
+// MI355X, us per call of the whole op, one sequence of 8 v-heads: 4,096 tokens
+// 174.9 -> 74.1, 32,768 tokens 1266 -> 276; 4 ragged sequences of 8,192
+// tokens in all, 16 v-heads: 173 -> 142.  A batch that is offered the passes
+// but keeps whole sequences pays about 4 us for the two idle launches.
+//
+// A transition entry outside [-kSegLimit, kSegLimit] (or NaN) makes the whole
+// head run in order: with keys of norm <= 1, beta in [0, 1] and decays <= 1 a
+// transition has norm <= 1 and its products lose nothing; without these they
+// could overflow or cancel where the chain in order does not.
+// ---------------------------------------------------------------------------
+constexpr float kSegLimit = 2.f;
+constexpr int64_t kSegImg = 128 * 128 * 4;  // bf16 hi and lo images of one transition
+constexpr int64_t kSegSeqs = 16;            // most sequences (the plan loops over them)
+
+// Time of the state pass (us) when the longest sequence is cut into `s`
+// segments of `len` chunks: `sums` kSegSum blocks and `outs` kSegOut blocks,
+// each on one CU at a time.  A step takes 1.6 (sum) or 2.35 us (out) on an
+// idle chip and about 0.6 us more on a full one, a step of the combine
+// kernel 1.2 us (measured on MI355X; the model is within 5% of the measured
+// passes from 2,048 to 32,768 tokens).  `exact`: the block counts are known,
+// so that a round of blocks that is nearly empty counts as one.
+__host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, int cus,
+                                          bool exact) {
+  auto time = [&](int blocks, float step) {
+    const float load = static_cast<float>(blocks) / cus;
+    return fmaxf(1.f, exact ? ceilf(load) : load) * len * (step + 0.6f * fminf(1.f, load));
+  };
+  const float out = 8.f + time(outs, 2.35f);
+  return s <= 1 ? out : out + 14.f + time(sums, 1.6f) + 1.2f * (s - 2);
+}
+
+// Chunks per segment for this batch, 0 for whole sequences (wave-uniform; N <=
+// kSegSeqs).
+__device__ __forceinline__ int wave_seg_len(const ChunkParams& p) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int N = static_cast<int>(p.N);
+  const WaveSeqs w = wave_seqs(p);
+  int longest = 1;
+  for (int n = 0; n < N; ++n) longest = max(longest, __builtin_amdgcn_readlane(w.cnt, n));
+  const int len = (longest + lane) / (lane + 1);
+  int segs = 0, ms = 0;
+  for (int n = 0; n < N; ++n) {
+    const int c = (__builtin_amdgcn_readlane(w.cnt, n) + len - 1) / len;
+    segs += max(c, 1);
+    ms += max(c - 2, 0);
+  }
+  const float cost = seg_cost(lane + 1, len, ((segs - N) * p.seg_nvt + ms * 2) * p.HV,
+                              segs * p.seg_nvt * p.HV, p.seg_cus, true);
+  // Smallest cost, the fewest segments among equals.
+  int key = lane == 0 || segs <= p.seg_max ? static_cast<int>(fminf(cost * 16.f, 3e7f)) : 30000000;
+  key = key * kWave + lane;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) key = min(key, __shfl_xor(key, o, kWave));
+  const int best = __builtin_amdgcn_readfirstlane(key & (kWave - 1));
+  return best ? __builtin_amdgcn_readlane(len, best) : 0;
+}
+
+struct WaveSegs {
+  WaveSeqs s;
+  int len;       // chunks per segment, 0: whole sequences
+  int32_t cnt;   // sequence lane's segments (an empty sequence has one)
+  int32_t incl;  // segments of sequences 0 .. lane
+};
+__device__ __forceinline__ WaveSegs wave_segs(const ChunkParams& p) {
+  WaveSegs w;
+  w.len = *p.seg_len;
+  w.s = wave_seqs(p);
+  const int lane = threadIdx.x & (kWave - 1);
+  w.cnt = lane >= p.N ? 0 : w.len ? max((w.s.cnt + w.len - 1) / w.len, 1) : 1;
+  w.incl = wave_incl_scan(w.cnt);
+  return w;
 }
 
 // Rows >= L of the K / Q operands (q4_load) repeat row L-1; here every
@@ -153,6 +255,11 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   const int hg4 = (p.HV + 3) >> 2;
   const int64_t c = blockIdx.x / hg4;
   const int hv = static_cast<int>(blockIdx.x % hg4) * 4 + wid;
+  if (c == p.NTmax) {  // the one block past the chunks (launched with seg_max)
+    const int len = wave_seg_len(p);
+    if (threadIdx.x == 0) *p.seg_len = len;
+    return;
+  }
   int64_t s;
   int L;
   if (p.N <= kWaveSeqs) {
@@ -684,6 +791,10 @@ gdn_chunk_state_kernel(ChunkParams p, int nvt) {
 // ---------------------------------------------------------------------------
 constexpr int kTh8 = 512;
 
+// Modes of the 64-column state kernel: whole sequences, or (segments of a
+// sequence in parallel) end states and transitions only, then outputs.
+enum { kSegNone = 0, kSegSum = 1, kSegOut = 2 };
+
 // The transposed tiles below (sb8_off, t8_off) are unpadded and swizzled.
 
 template <int K>
@@ -711,7 +822,7 @@ struct OutOps8 {
 };
 typedef __attribute__((address_space(4))) const float cfloat_t;
 
-template <int K>
+template <int K, int MODE>
 __global__ void __launch_bounds__(kTh8) __attribute__((amdgpu_waves_per_eu(2)))
 gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   constexpr int BV = 64;
@@ -719,6 +830,7 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   __shared__ P2Smem8<K> sm;
   constexpr int KK = K / 32;
   constexpr int NJ = 2;  // 16-column tiles per wave
+  constexpr bool kOut = MODE != kSegSum;
   const int tid = threadIdx.x;
   const int wid = wave_index();
   // Waves w and w + 4 share a SIMD; they take token rows wr and 3 - wr, so
@@ -731,17 +843,70 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   const int rl = lane >> 4, ch = lane & 15;  // whole-row loads: row in a load, 16-byte chunk
   const int64_t w = blockIdx.x;
   const int64_t xcd = w & 7, r = w >> 3;
-  const int vt = static_cast<int>(r % nvt);
-  const int64_t item = (r / nvt) * 8 + xcd;
-  if (item >= p.N * p.HV) return;
-  int64_t n, cidx0;
-  find_ranked_seq(p, item / p.HV, n, cidx0);
+  const int ntile = MODE == kSegSum ? nvt + K / 64 : nvt;
+  const int vt = static_cast<int>(r % ntile);
+  const int64_t item = (r / ntile) * 8 + xcd;
   const int hv = state_head(static_cast<int>(item % p.HV), p.HV, p.H);
   const int hq = hv / (p.HV / p.H);
   const int V = nvt * BV;
-  const int v0 = vt * BV;
-  const int64_t bos = cu_at(p, n), eos = cu_at(p, n + 1);
-  const int64_t nch = max<int64_t>(0, min<int64_t>((eos - bos + kC - 1) / kC, p.NTmax - cidx0));
+  const bool is_m = MODE == kSegSum && vt >= nvt;  // block of the transition's columns
+  const int v0 = is_m ? 0 : vt * BV;
+  int64_t n, cidx0, bos, eos, nch;
+  // Where the state comes from (NULL: zero) and goes to (NULL: nowhere).
+  const float* s_in;
+  float* s_out;
+  int64_t sh = 0;  // (segment, head)
+  int before = 0;  // segments of the sequence before this one
+  if constexpr (MODE == kSegNone) {
+    if (item >= p.N * p.HV) return;
+    find_ranked_seq(p, item / p.HV, n, cidx0);
+    bos = cu_at(p, n);
+    eos = cu_at(p, n + 1);
+    nch = (eos - bos + kC - 1) / kC;
+    const int64_t at = (n * p.HV + hv) * K * V;
+    s_in = p.h0 ? p.h0 + at : nullptr;
+    s_out = p.ht ? p.ht + at : nullptr;
+  } else {
+    if (MODE == kSegSum && !*p.seg_len) return;  // (with 1 block a CU, idle ones should be short)
+    const WaveSegs ws = wave_segs(p);
+    // kSegSum blocks skip the last segment of every sequence: its end state
+    // is not needed.
+    const int skip = MODE == kSegSum ? (lane < p.N ? lane + 1 : static_cast<int>(p.N)) : 0;
+    const int64_t at_seg = item / p.HV;
+    if (at_seg >= __builtin_amdgcn_readlane(ws.incl - skip, kWave - 1)) return;
+    const int nn = __popcll(__ballot(ws.incl - skip <= at_seg));
+    n = nn;
+    const int cnt = __builtin_amdgcn_readlane(ws.cnt, nn);
+    const int64_t seg = at_seg + (MODE == kSegSum ? nn : 0);
+    if (seg >= p.seg_max) return;
+    before = static_cast<int>(seg) - (__builtin_amdgcn_readlane(ws.incl, nn) - cnt);
+    const int first = before * ws.len;  // chunk of the sequence
+    sh = seg * p.HV + hv;
+    cidx0 = __builtin_amdgcn_readlane(ws.s.incl - ws.s.cnt, nn) + first;
+    bos = readlane64(ws.s.a, nn) + static_cast<int64_t>(first) * kC;
+    eos = readlane64(ws.s.b, nn);
+    nch = __builtin_amdgcn_readlane(ws.s.cnt, nn) - first;
+    if (ws.len) nch = min(nch, ws.len);
+    const int64_t at = (n * p.HV + hv) * K * V;
+    s_in = p.h0 ? p.h0 + at : nullptr;
+    if constexpr (MODE == kSegSum) {
+      if (is_m && before == 0) return;  // the first segment's transition is not needed
+      if (before > 0) s_in = nullptr;
+      s_out = is_m ? nullptr : p.seg_b + sh * K * V;
+    } else {
+      const bool in_order = cnt > 1 && p.seg_bad[n * p.HV + hv] != 0;
+      if (in_order) {
+        if (before > 0) return;
+        nch = __builtin_amdgcn_readlane(ws.s.cnt, nn);
+      }
+      if (before > 0) s_in = p.seg_b + (sh - p.HV) * K * V;
+      s_out = p.ht && (in_order || before == cnt - 1) ? p.ht + at : nullptr;
+    }
+  }
+  // The NTmax bound keeps a malformed cu_seqlens (never a well-formed one)
+  // from reading past the workspace.
+  nch = max<int64_t>(0, min<int64_t>(nch, p.NTmax - cidx0));
+  const int scol = is_m ? (vt - nvt) * BV : vt * BV;  // first column of the state block
 
   constexpr int M2 = K / 64;
   f4_t sreg[M2][NJ];
@@ -752,8 +917,9 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int kr = wr * (K / 4) + m2 * 16 + 4 * lg + i;
-        sreg[m2][nj][i] =
-            p.h0 ? p.h0[((n * p.HV + hv) * K + kr) * V + v0 + cb + nj * 16 + l15] : 0.f;
+        const int col = scol + cb + nj * 16 + l15;
+        if (is_m) sreg[m2][nj][i] = kr == col ? 1.f : 0.f;
+        else sreg[m2][nj][i] = s_in ? s_in[static_cast<int64_t>(kr) * V + col] : 0.f;
       }
   auto publish_state = [&]() {
 #pragma unroll
@@ -780,12 +946,13 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     for (int j = 0; j < 2; ++j) {
       const uint32_t off = static_cast<uint32_t>(min(wr * 16 + cg * 8 + 4 * j + rl, L - 1)) * rb + 16u * ch;
       o.kraw[j] = *reinterpret_cast<const bf8_t*>(kb + off);
-      o.qraw[j] = *reinterpret_cast<const bf8_t*>(qb + off);
+      if constexpr (kOut) o.qraw[j] = *reinterpret_cast<const bf8_t*>(qb + off);
     }
     const WaveRows wrs = wave_rows(s, L, wr);
     const char* vb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.v) +
                                                    wrs.row0 * vrow + vcol0);
     o.vA = *reinterpret_cast<const bf8_t*>(vb + row_off(l15, wrs.lw, 2 * vrow, 8 * lg));
+    if (is_m) o.vA = bf8_t{};  // a transition has no values (and takes no NaN from them)
     // The factor block (cq, ck, beta, ed: 1 KB) in one load per wave; the
     // wave-uniform e^{g_last} through the scalar cache.
     const char* sc = rec_at(p, cidx, hv) + 3 * kMat;
@@ -824,9 +991,9 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     __builtin_amdgcn_sched_barrier(0);
     load_inv8(inv, cidx0);
     __builtin_amdgcn_sched_barrier(0);
-    load_out8(outo, cidx0);
+    if constexpr (kOut) load_out8(outo, cidx0);
     store_rows(sm.kr[0], opsA.kraw);
-    store_rows(sm.qr, opsA.qraw);
+    if constexpr (kOut) store_rows(sm.qr, opsA.qraw);
     store_fac(sm.fac[0], opsA.fac);
   }
   __syncthreads();
@@ -897,13 +1064,15 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
         d[i] = ed[i] * vn[nj][i];
       }
       split4(d, h, l);
-      *reinterpret_cast<Vec<__bf16, 4>*>(&sm.vt[t8_off(cb + nj * 16 + l15, wr * 16 + 4 * lg)]) = b;
+      if constexpr (kOut)
+        *reinterpret_cast<Vec<__bf16, 4>*>(&sm.vt[t8_off(cb + nj * 16 + l15, wr * 16 + 4 * lg)]) = b;
       *reinterpret_cast<Vec<__bf16, 4>*>(&sm.dt[0][t8_off(cb + nj * 16 + l15, wr * 16 + 4 * lg)]) = h;
       *reinterpret_cast<Vec<__bf16, 4>*>(&sm.dt[1][t8_off(cb + nj * 16 + l15, wr * 16 + 4 * lg)]) = l;
     }
     load_inv8(inv, cidx0 + cn);
     // (Q S)^T = S^T Q^T: Q's rows from the query tile, keys in natural order.
     f4_t qs[NJ];
+    if constexpr (kOut) {
 #pragma unroll
     for (int nj = 0; nj < NJ; ++nj) qs[nj] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -915,9 +1084,10 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
         qs[nj] = mfma16(sh, qa, qs[nj]);
       }
     }
+    }
     __syncthreads();  // (2) vt, dt complete; rt, sb and query reads done
 
-    {
+    if constexpr (kOut) {
       const int row = wr * 16 + quad_row(), qb = quad_col();
       const float cq = fc[0 * kC + wr * 16 + l15];
       bf16* orow = row < L ? reinterpret_cast<bf16*>(p.o) + static_cast<uint64_t>(s + row) * vrow + vcol0
@@ -939,7 +1109,7 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
         *reinterpret_cast<u32x2*>(orow + nj * 16 + 4 * qb) = quad_rows(__builtin_bit_cast(u32x2, ov));
       }
     }
-    load_out8(outo, cidx0 + cn);
+    if constexpr (kOut) load_out8(outo, cidx0 + cn);
 
     __builtin_amdgcn_iglp_opt(0);
 #pragma unroll
@@ -965,7 +1135,7 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     }
     publish_state();
     store_rows(sm.kr[(ci + 1) & 1], nxt.kraw);
-    store_rows(sm.qr, nxt.qraw);
+    if constexpr (kOut) store_rows(sm.qr, nxt.qraw);
     store_fac(sm.fac[(ci + 1) & 1], nxt.fac);
     __syncthreads();  // (3)
   };
@@ -973,7 +1143,26 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     step(opsA, opsB, ci);
     if (ci + 1 < nch) step(opsB, opsA, ci + 1);
   }
-  if (p.ht) {
+  if (is_m) {
+    // Transition columns scol .. + 63 as A operands of the combine kernel
+    // (image (w, kk), hi then lo: rows 16 w + l % 16, columns 32 kk + 8 (l /
+    // 16) .. + 7), read transposed from the state's bf16 copy.
+    bool over = false;
+    char* img = p.seg_m + sh * kSegImg + (wid * KK + scol / 32) * 2048 + 16 * lane;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int r0 = 32 * kk + 8 * lg;
+        const bf8_t x = cat_bf8(sb8_col4(sm.sb[h], 16 * wid, r0), sb8_col4(sm.sb[h], 16 * wid, r0 + 4));
+        *reinterpret_cast<bf8_t*>(img + 2048 * kk + 1024 * h) = x;
+        if (h == 0)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) over |= !(fabsf(static_cast<float>(x[e])) <= kSegLimit);
+      }
+    const int any = __syncthreads_or(over);
+    if (tid == 0) p.seg_over[2 * sh + (vt - nvt)] = any;
+  } else if (s_out) {
 #pragma unroll
     for (int m2 = 0; m2 < M2; ++m2)
 #pragma unroll
@@ -981,9 +1170,124 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int kr = wr * (K / 4) + m2 * 16 + 4 * lg + i;
-          p.ht[((n * p.HV + hv) * K + kr) * V + v0 + cb + nj * 16 + l15] = sreg[m2][nj][i];
+          s_out[static_cast<int64_t>(kr) * V + scol + cb + nj * 16 + l15] = sreg[m2][nj][i];
         }
   }
+}
+
+
+// ---------------------------------------------------------------------------
+// States at the segment boundaries of one (sequence, v-head, 16 V columns):
+// S_1 = the state after segment 0, S_{i+1} = M_i S_i + B_i; S_{i+1} replaces
+// B_i.  A block of eight waves; wave w owns state rows 16 w .. + 15.  A step
+// is bound by its 64 KB of operand images into one CU and takes 1.2 us
+// (2.2 us with M in fp32, split here by every column tile; as a prologue of
+// the kSegOut blocks, whose 64 columns need each image in two waves, 2.5 us).
+// ---------------------------------------------------------------------------
+template <int K>
+__global__ void __launch_bounds__(kTh8) gdn_chunk_combine_kernel(ChunkParams p, int V) {
+  static_assert(K == 128, "eight waves of 16 rows");
+  constexpr int KK = K / 32;
+  constexpr int kDepth = 3;  // steps whose operands are in flight
+  __shared__ __align__(16) __bf16 sb[2][2][16 * K];  // state hi / lo [v][k], double-buffered
+  const int lane = threadIdx.x & 63, wid = wave_index();
+  const int l15 = lane & 15, lg = lane >> 4;
+  const int nt = V / 16;
+  // The column tiles of one head read the same transitions: on one XCD.
+  const int64_t xcd = blockIdx.x & 7, r = blockIdx.x >> 3;
+  const int v0 = static_cast<int>(r % nt) * 16;
+  const int64_t item = (r / nt) * 8 + xcd;
+  if (item >= p.N * p.HV) return;
+  if (!*p.seg_len) return;
+  const int hv = static_cast<int>(item % p.HV);
+  const WaveSegs ws = wave_segs(p);
+  const int nn = static_cast<int>(item / p.HV);
+  const int seg0 = __builtin_amdgcn_readlane(ws.incl - ws.cnt, nn);
+  const int cnt = min(__builtin_amdgcn_readlane(ws.cnt, nn), p.seg_max - seg0);
+  if (cnt <= 1) return;  // no boundary
+  const int64_t sh0 = static_cast<int64_t>(seg0) * p.HV + hv;
+  if (v0 == 0 && wid == 0) {
+    int over = 0;
+    for (int i = lane; i < 2 * (cnt - 2); i += kWave)
+      over |= p.seg_over[2 * (sh0 + (1 + (i >> 1)) * static_cast<int64_t>(p.HV)) + (i & 1)];
+    const uint64_t any = __ballot(over != 0);
+    if (lane == 0) p.seg_bad[item] = any != 0;
+  }
+  const int r4 = 16 * wid + 4 * lg;  // first of the lane's four state rows
+  // Per-step strides and the lane's place in each, so that a step's
+  // addresses are one scalar base plus one lane offset.
+  float* bseg = p.seg_b + sh0 * K * V;
+  const int64_t bstep = static_cast<int64_t>(p.HV) * K * V;
+  const uint32_t boff = static_cast<uint32_t>(r4) * V + v0 + l15;
+  const char* mseg = p.seg_m + sh0 * kSegImg + wid * (2 * KK * 1024);
+  const int64_t mstep = static_cast<int64_t>(p.HV) * kSegImg;
+  struct Stage {
+    bf8_t mh[KK], ml[KK];
+    f4_t b;
+  } st[kDepth];
+  auto load_b = [&](int i) {
+    const float* b = bseg + i * bstep;
+    return f4_t{b[boff], b[boff + V], b[boff + 2 * V], b[boff + 3 * V]};
+  };
+  auto load = [&](Stage& t, int i) {
+    t.b = load_b(i);
+    const char* m = mseg + i * mstep;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      t.mh[kk] = *reinterpret_cast<const bf8_t*>(m + 2048 * kk + 16u * lane);
+      t.ml[kk] = *reinterpret_cast<const bf8_t*>(m + 2048 * kk + 1024 + 16u * lane);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto store = [&](int i, const f4_t& v) {
+    float* out = bseg + i * bstep;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[boff + e * V] = v[e];
+  };
+  // Loads and stores count in one in-order counter, so a wait for a load
+  // waits for everything issued before it: every load of the loop is
+  // unconditional (past the last step it repeats that step's, unused), in
+  // the order the steps take them, and a step stores the state it starts
+  // from, ahead of its loads.
+  const int last = cnt - 2;
+  f4_t s = load_b(0);
+  __builtin_amdgcn_sched_barrier(0);
+  if (last > 0) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) load(st[u], min(u + 1, last));
+  }
+  auto step = [&](Stage& t, int i) {
+    const int buf = i & 1;
+    Vec<__bf16, 4> h, l;
+    split4(s, h, l);
+    *reinterpret_cast<Vec<__bf16, 4>*>(&sb[buf][0][sb8_off(l15, r4)]) = h;
+    *reinterpret_cast<Vec<__bf16, 4>*>(&sb[buf][1][sb8_off(l15, r4)]) = l;
+    store(i - 1, s);
+    // State copy complete; the other buffer's readers passed the barrier before.
+    __syncthreads();
+    f4_t c = {0.f, 0.f, 0.f, 0.f};
+    s = t.b;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      const bf8_t sh = *reinterpret_cast<const bf8_t*>(&sb[buf][0][sb8_off(l15, 32 * kk + 8 * lg)]);
+      const bf8_t sl = *reinterpret_cast<const bf8_t*>(&sb[buf][1][sb8_off(l15, 32 * kk + 8 * lg)]);
+      s = mfma16(t.mh[kk], sh, s);
+      c = mfma16(t.mh[kk], sl, c);
+      c = mfma16(t.ml[kk], sh, c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load(t, min(i + kDepth, last));
+    s += c;
+  };
+  int i = 1;
+  for (; i + kDepth - 1 <= last; i += kDepth) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) step(st[u], i + u);
+  }
+#pragma unroll
+  for (int u = 0; u < kDepth - 1; ++u)
+    if (i + u <= last) step(st[u], i + u);
+  if (last > 0) store(last, s);
 }
 
 template <int K, typename GT, typename BT>
@@ -995,16 +1299,30 @@ int launch_chunk(const ChunkParams& p, int64_t V, hipStream_t s) {
     if ((st = launch_status())) return st;
   }
   const int64_t prep_blocks = p.NTmax * ((p.HV + 3) / 4);
-  if (prep_blocks > INT32_MAX) return XK_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL((gdn_chunk_prep_kernel<K, GT, BT>), dim3(static_cast<uint32_t>(prep_blocks)),
+  if (prep_blocks >= INT32_MAX) return XK_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL((gdn_chunk_prep_kernel<K, GT, BT>),
+                     dim3(static_cast<uint32_t>(prep_blocks) + (p.seg_max ? 1 : 0)),
                      dim3(kTh), 0, s, p);
   st = launch_status();
   if (st) return st;
   const int64_t items = p.N * p.HV;
-  if (V % 64 == 0) {
+  if (V % 64 == 0 && p.seg_max > 0) {
+    const int nvt = static_cast<int>(V / 64);
+    const int64_t seg_items = cdiv(static_cast<int64_t>(p.seg_max) * p.HV, 8) * 8;
+    const int64_t sum_items = cdiv((p.seg_max - p.N) * p.HV, 8) * 8;
+    hipLaunchKernelGGL((gdn_chunk_state8_kernel<K, kSegSum>), dim3(sum_items * (nvt + K / 64)),
+                       dim3(kTh8), 0, s, p, nvt);
+    if ((st = launch_status())) return st;
+    hipLaunchKernelGGL((gdn_chunk_combine_kernel<K>), dim3(cdiv(items, 8) * 8 * (V / 16)),
+                       dim3(kTh8), 0, s, p, static_cast<int>(V));
+    if ((st = launch_status())) return st;
+    hipLaunchKernelGGL((gdn_chunk_state8_kernel<K, kSegOut>), dim3(seg_items * nvt), dim3(kTh8), 0,
+                       s, p, nvt);
+  } else if (V % 64 == 0) {
     const int nvt = static_cast<int>(V / 64);
     const int64_t blocks = cdiv(items, 8) * 8 * nvt;
-    hipLaunchKernelGGL((gdn_chunk_state8_kernel<K>), dim3(blocks), dim3(kTh8), 0, s, p, nvt);
+    hipLaunchKernelGGL((gdn_chunk_state8_kernel<K, kSegNone>), dim3(blocks), dim3(kTh8), 0, s, p,
+                       nvt);
   } else {
     constexpr int BV = 32;
     const int nvt = static_cast<int>(V / BV);
@@ -1025,17 +1343,67 @@ int chunk_beta(const ChunkParams& p, int64_t V, xk_dtype bdt, hipStream_t s) {
 
 int64_t nt_max(int64_t total_tokens, int64_t N) { return total_tokens / kC + N; }
 
+// Whether a call takes the segmented state pass, and its workspace past the
+// records.  The lengths are not known here: several sequences are taken to
+// be ragged (the longest 1.5 times their mean), one is known exactly.
+struct SegPlan {
+  int segs = 0;  // most segments; 0: whole sequences
+  int64_t bytes = 0;
+};
+SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t V) {
+  SegPlan r;
+  const int cus = num_cus();
+  const int64_t tiles = HV * (V / 64);
+  // Several sequences that fill over half the chip leave no whole round of
+  // blocks to gain (3 sequences of 32 v-heads: 409 us without, 433 with).
+  if (N <= 0 || N > kSegSeqs || V % 64 != 0 || N * tiles * (N > 1 ? 2 : 1) > cus) return r;
+  const int64_t chunks = cdiv(total_tokens, kC);
+  const int64_t longest = N == 1 ? chunks : cdiv(3 * chunks, 2 * N);
+  auto cost = [&](int s, int64_t len, int64_t sums, int64_t outs) {
+    return seg_cost(s, static_cast<int>(len), static_cast<int>(std::max<int64_t>(sums, 0)),
+                    static_cast<int>(outs), cus, N == 1);
+  };
+  float best = cost(1, longest, 0, N * tiles);
+  if (N > 1) best -= 4.f;  // what the passes cost a batch that turns out not to gain
+  for (int s = 2; s <= 64; ++s) {
+    const int64_t len = cdiv(longest, s);
+    const int64_t segs = N == 1 ? cdiv(chunks, len) : chunks / len + N / 2;
+    const int64_t sums = (segs - N) * (tiles + 2 * HV) - (N == 1 ? 2 : N) * HV;
+    const float c = cost(s, len, sums, segs * tiles);
+    if (c < best) {
+      best = c;
+      r.segs = static_cast<int>(segs);
+    }
+  }
+  // Several sequences: room for one round of kSegOut blocks.
+  if (r.segs && N > 1) r.segs = static_cast<int>(std::max<int64_t>(r.segs, cus / tiles) + N / 2);
+  if (r.segs)
+    r.bytes = 256 + align256(4 * N * HV) + align256(8 * r.segs * HV) +
+              r.segs * HV * (kSegImg + K * V * 4);
+  return r;
+}
+
 }  // namespace
 }  // namespace xk
 
 using namespace xk;
 
+namespace {
+
+// The least a call runs in (without segments).
+int64_t least_workspace(int64_t total_tokens, int64_t N, int64_t HV) {
+  const int64_t nt = nt_max(total_tokens, N);
+  return align256(4 * (N + 1)) + align256(4 * N) + align256(8 * nt) + kDump + nt * HV * kRec;
+}
+
+}  // namespace
+
 extern "C" int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                                 int64_t HV) {
   if (total_tokens < 0 || num_seqs < 0 || HV <= 0) return -1;
-  const int64_t nt = nt_max(total_tokens, num_seqs);
-  return align256(4 * (num_seqs + 1)) + align256(4 * num_seqs) + align256(8 * nt) + kDump +
-         nt * HV * kRec;
+  // Room for the segments of 128 x 128 states; wider ones run without.
+  return least_workspace(total_tokens, num_seqs, HV) +
+         seg_plan(total_tokens, num_seqs, HV, 128, 128).bytes;
 }
 
 namespace xk {
@@ -1088,7 +1456,7 @@ extern "C" int xk_gdn_chunk_fwd(
   const int ast = chunk_args_status(q, k, v, dtype, g, g_dtype, beta, beta_dtype, o, cu_seqlens,
                                     cu_dtype, N, total_tokens, H, HV, K, V, &empty);
   if (ast != XK_OK || empty) return ast;
-  const int64_t need = xk_gdn_chunk_workspace_bytes(total_tokens, N, HV);
+  const int64_t need = least_workspace(total_tokens, N, HV);
   if (!workspace || static_cast<int64_t>(workspace_bytes) < need) return XK_ERR_WORKSPACE;
   if (!aligned(workspace, 256)) return XK_ERR_WORKSPACE;
   ChunkParams p{};
@@ -1118,6 +1486,21 @@ extern "C" int xk_gdn_chunk_fwd(
   p.HV = static_cast<int>(HV);
   p.scale = scale;
   p.l2norm = use_qk_l2norm;
+  const SegPlan plan = seg_plan(total_tokens, N, HV, K, V);
+  if (plan.segs && static_cast<int64_t>(workspace_bytes) >= need + plan.bytes) {
+    char* seg = p.rec + p.NTmax * HV * kRec;
+    p.seg_max = plan.segs;
+    p.seg_cus = num_cus();
+    p.seg_nvt = static_cast<int>(V / 64);
+    p.seg_len = reinterpret_cast<int32_t*>(seg);
+    seg += 256;
+    p.seg_bad = reinterpret_cast<int32_t*>(seg);
+    seg += align256(4 * N * HV);
+    p.seg_over = reinterpret_cast<int32_t*>(seg);
+    seg += align256(8 * plan.segs * HV);
+    p.seg_m = seg;
+    p.seg_b = reinterpret_cast<float*>(seg + plan.segs * HV * kSegImg);
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (g_dtype == XK_F32) return chunk_beta<128, float>(p, V, beta_dtype, s);
   return chunk_beta<128, bf16>(p, V, beta_dtype, s);
@@ -1181,8 +1564,7 @@ extern "C" int xk_gdn_chunk_fwd_noalloc(
   const int ast = chunk_args_status(q, k, v, dtype, g, g_dtype, beta, beta_dtype, o, cu_seqlens,
                                     cu_dtype, N, total_tokens, H, HV, K, V, &empty);
   if (ast != XK_OK || empty) return ast;
-  const int64_t need = xk_gdn_chunk_workspace_bytes(total_tokens, N, HV);
-  if (need < 0) return XK_ERR_INVALID;
+  const int64_t need = least_workspace(total_tokens, N, HV);
   if (need > kNoAllocScratchBytes) return XK_ERR_SCRATCH;
   void* ws = nullptr;
   const int st = scratch_on_current_device(static_cast<hipStream_t>(stream), &ws);

@@ -60,10 +60,8 @@ __device__ __forceinline__ void split4(const f4_t& x, Vec<__bf16, 4>& h, Vec<__b
   l.v[3] = l1[1];
 }
 
-// Eight consecutive fp32 values (16-byte aligned) split into hi / lo.
-__device__ __forceinline__ void split8(const float* p, bf8_t& h, bf8_t& l) {
-  const f4_t a = *reinterpret_cast<const f4_t*>(p);
-  const f4_t b = *reinterpret_cast<const f4_t*>(p + 4);
+// Eight values split into hi / lo.
+__device__ __forceinline__ void split8(const f4_t& a, const f4_t& b, bf8_t& h, bf8_t& l) {
 #pragma unroll
   for (int e = 0; e < 4; e += 2) {
     bf2_t x, y;
@@ -78,6 +76,10 @@ __device__ __forceinline__ void split8(const float* p, bf8_t& h, bf8_t& l) {
     l[e + 4] = y[0];
     l[e + 5] = y[1];
   }
+}
+// Eight consecutive fp32 values (16-byte aligned) split into hi / lo.
+__device__ __forceinline__ void split8(const float* p, bf8_t& h, bf8_t& l) {
+  split8(*reinterpret_cast<const f4_t*>(p), *reinterpret_cast<const f4_t*>(p + 4), h, l);
 }
 
 // B operand that selects columns 16h .. 16h + 15 of a 32-wide A operand:
