@@ -276,3 +276,46 @@ def test_v2_history_read_next_to_a_tile_edge(dev, W):
                                               slots.to(dev), qsl.to(dev), 33, state_rule=rule)
         torch.testing.assert_close(out.float().cpu(), ref, **BF16_TOL)
         assert torch.equal(st_d.cpu(), ref_state.to(torch.bfloat16))
+
+
+# Batches of short sequences (one lane per sequence and channel pair): empty
+# and one-token sequences, lengths around the groups of four tokens and the
+# longest one sent there (32, and 33 past it); whole and partial 512-channel
+# blocks and odd channel counts; states contiguous, with channels apart, and
+# token-major; speculative windows and a padded slot.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("spec", [False, True])
+@pytest.mark.parametrize("layout", ["dense", "apart", "token_major"])
+@pytest.mark.parametrize("lens,dim,W", [
+    ([1] * 9, 1024, 4), ([4, 4, 4], 1030, 4), ([0, 1, 3, 5, 4, 8, 0], 513, 4),
+    ([32, 1, 31], 512, 4), ([33, 2], 512, 4), ([2, 3, 1], 520, 2), ([5, 6], 200, 6),
+    ([3, 1], 7, 1)])
+def test_v2_short_sequences(dev, lens, dim, W, layout, spec, dtype):
+    from torch_npu_ops_amd import ops
+    g = torch.Generator().manual_seed(sum(lens) + dim)
+    B, longest = len(lens), max(lens)
+    S = max(W - 1 + (longest - 1 if spec else 0), 1)
+    lines = B + 3
+    state = _rn((lines, dim, S), g, dtype)
+    x = _rn((sum(lens), dim), g, dtype)
+    w, b = _rn((dim, W), g, dtype), _rn((dim,), g, dtype)
+    slots = torch.randperm(lines, generator=g)[:B].to(torch.int32)
+    if B > 2:
+        slots[1] = -1  # padded
+    qsl = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    acc = torch.tensor([max(1, n - i % 2) for i, n in enumerate(lens)], dtype=torch.int32) if spec else None
+    ref, ref_state = oc.causal_conv1d_update_v2(x, state, w, b, True, slots, qsl, longest,
+                                                num_accepted_tokens=acc)
+    if layout == "dense":
+        st = state.to(dev)
+    elif layout == "apart":
+        st = torch.zeros(lines, dim, S + 3, dtype=dtype, device=dev)[:, :, :S]
+        st.copy_(state)
+    else:
+        st = state.to(dev).transpose(1, 2).contiguous().transpose(1, 2)
+    out = ops.npu_causal_conv1d_update_v2(
+        x.to(dev), st, w.to(dev), True, b.to(dev), slots.to(dev), qsl.to(dev), longest,
+        num_accepted_tokens=acc.to(dev) if spec else None)
+    live = torch.cat([torch.full((n,), bool(s != -1)) for n, s in zip(lens, slots)])
+    torch.testing.assert_close(out.float().cpu()[live], ref[live], **_tol(dtype))
+    assert torch.equal(st.cpu(), ref_state.to(dtype))

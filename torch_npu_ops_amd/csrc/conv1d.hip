@@ -229,6 +229,7 @@ struct VarlenParams {
   int state_rule;  // 0: reference rule, 1: prefill rule
   int silu_on;
   int32_t pad;
+  int short_stage;  // conv1d_short_kernel moves states through LDS
   int w_vec;  // weights are [D, W] contiguous, x's dtype, 16-byte aligned
   int64_t ncb, ntt;  // prefill grid: channel blocks x token tiles
 };
@@ -515,6 +516,173 @@ __global__ void __launch_bounds__(256) conv1d_varlen_kernel(VarlenParams p) {
     if (p.qsl[sq] >= t0) write_state(sq);
 }
 
+// ---------------------------------------------------------------------------
+// Varlen batches of short sequences (speculative verification, decode through
+// the varlen entry): one lane per (sequence, VEC channels), which loads the
+// window, the state entries it keeps and the first tokens at once, walks its
+// tokens and writes the state.  The tile kernel above has one lane per (16
+// tokens, 8 channels): a few sequences' tokens fill a fraction of the CUs
+// there, and each lane gathers and scatters the 2-byte state entries of all
+// its sequences one after the other.  Bound by the chain slot -> state ->
+// output at small batches; at 256 sequences of 8 drafts by its bytes (70% of
+// a copy's rate).  MI355X, 8192 bf16 channels, width 4, us per call, tile
+// kernel -> this one (with direct state accesses in brackets):
+//   32 sequences of 1 token                142.3 -> 5.5 (5.7)
+//   32 of 4 tokens, speculative (6 entries) 75.0 -> 6.6 (8.2)
+//   256 of 8 tokens, speculative           213.2 -> 35.0 (79.5)
+// ---------------------------------------------------------------------------
+// Longest sequence (as the caller declares it) sent here: a lane walks it
+// alone.  One sequence of 32 tokens takes 9.1 us here and 13.7 in the tile
+// kernel, one of 64 takes 13.8 and 13.9 and is left there.
+constexpr int64_t kShortLen = 32;
+constexpr int64_t kShortLds = 32768;  // most LDS for a block's states
+constexpr int kShortTok = 4;   // tokens loaded together
+constexpr int kShortKeep = 8;  // kept state entries loaded together
+template <typename T, int W, int VEC, bool SILU>
+__global__ void __launch_bounds__(256) conv1d_short_kernel(VarlenParams p) {
+  using VT = Vec<T, VEC>;
+  extern __shared__ __align__(16) char short_lds[];
+  const int s = static_cast<int>(blockIdx.x / p.ncb);
+  const int64_t cb = static_cast<int64_t>(blockIdx.x % p.ncb) * 256 * VEC;
+  const int64_t c0 = cb + threadIdx.x * VEC;
+  // Block-uniform: every block but a partial last one stages.
+  const bool stage = p.short_stage && cb + 256 * VEC <= p.D;
+  if (c0 >= p.D) return;
+  const int64_t start = p.qsl[s], end = p.qsl[s + 1], len = end - start;
+  const int64_t t_end = min(min(end, static_cast<int64_t>(p.qsl[p.B])), p.num_tokens);
+  if (len <= 0 || start < 0) return;
+  const int64_t in_slot = resolve_slot(p, s, p.init_idx);
+  if (p.slots && in_slot == p.pad) return;
+  const int64_t out_slot = resolve_slot(p, s, p.last_idx);
+  const int64_t off = p.accepted ? p.accepted[s] - 1 : 0;
+  const bool in_ok = in_slot >= 0 && in_slot < p.lines && off >= 0;
+  const T* x = reinterpret_cast<const T*>(p.x) + start * p.sx + c0;
+  T* out = reinterpret_cast<T*>(p.out) + start * p.so + c0;
+  const T* src = reinterpret_cast<const T*>(p.state) + in_slot * p.ssl + c0 * p.ssd;
+  // Staged: the block's 256 * VEC channels hold S contiguous entries each, so
+  // their states move as one contiguous run of 16-byte vectors through LDS,
+  // where each lane gathers its own (and later scatters the new ones).
+  T* own = reinterpret_cast<T*>(short_lds) + threadIdx.x * VEC * p.S;
+  const int nvec = static_cast<int>(256 * VEC * p.S * sizeof(T) / 16);
+  if (stage && in_ok) {
+    const u32x4* g = reinterpret_cast<const u32x4*>(src - threadIdx.x * VEC * p.S);
+    for (int i = threadIdx.x; i < nvec; i += 256) reinterpret_cast<u32x4*>(short_lds)[i] = g[i];
+    __syncthreads();
+    src = own;
+  }
+
+  // History (zeros where its entries do not lie in a real slot).
+  float win[W > 1 ? W - 1 : 1][VEC];
+  const bool hist = in_ok && off + (W - 1) <= p.S;
+#pragma unroll
+  for (int j = 0; j < W - 1; ++j)
+#pragma unroll
+    for (int u = 0; u < VEC; ++u) win[j][u] = hist ? to_f32(src[u * p.ssd + (off + j) * p.sss]) : 0.f;
+  // Final state: `run` entries, the last inputs; a shorter sequence keeps
+  // entries of the old state ahead of its inputs (the rule of write_state in
+  // the tile kernel).
+  const int64_t run = p.state_rule == 0 ? p.eff_state_len - (p.max_query_len - len)
+                                        : p.eff_state_len;
+  const bool write = out_slot >= 0 && out_slot < p.lines && run > 0 && run <= p.S &&
+                     start + len <= p.num_tokens;
+  const int64_t keep = write && len < run ? run - len : 0;
+  const int64_t from = off + (p.accepted ? 1 : len);
+  const int64_t kept = in_ok ? min(keep, p.S - from) : 0;  // entries that exist
+  T old[kShortKeep][VEC];
+#pragma unroll
+  for (int i = 0; i < kShortKeep; ++i)
+#pragma unroll
+    for (int u = 0; u < VEC; ++u)
+      old[i][u] = i < kept ? src[u * p.ssd + (from + i) * p.sss] : from_f32<T>(0.f);
+
+  float wt[W][VEC], bs[VEC];
+#pragma unroll
+  for (int u = 0; u < VEC; ++u) {
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+      wt[j][u] = p.w_vec ? to_f32(reinterpret_cast<const T*>(p.w)[(c0 + u) * W + j])
+                         : load_as_f32(p.w, (c0 + u) * p.swd + j * p.sww, p.wdt);
+    bs[u] = p.bias ? load_as_f32(p.bias, c0 + u, p.wdt) : 0.f;
+  }
+
+  const int64_t n = t_end - start;
+  for (int64_t t = 0; t < n; t += kShortTok) {
+    VT xs[kShortTok];
+#pragma unroll
+    for (int k = 0; k < kShortTok; ++k)
+      xs[k] = *reinterpret_cast<const VT*>(x + min(t + k, n - 1) * p.sx);
+#pragma unroll
+    for (int k = 0; k < kShortTok; ++k) {
+      if (t + k >= n) break;
+      VT ov;
+#pragma unroll
+      for (int u = 0; u < VEC; ++u) {
+        const float xc = to_f32(xs[k].v[u]);
+        float acc = bs[u];
+#pragma unroll
+        for (int j = 0; j < W - 1; ++j) acc = fmaf(win[j][u], wt[j][u], acc);
+        acc = fmaf(xc, wt[W - 1][u], acc);
+        if constexpr (SILU) acc = silu(acc);
+        ov.v[u] = from_f32<T>(acc);
+#pragma unroll
+        for (int j = 0; j + 1 < W - 1; ++j) win[j][u] = win[j + 1][u];
+        if constexpr (W > 1) win[W - 2][u] = xc;
+      }
+      *reinterpret_cast<VT*>(out + (t + k) * p.so) = ov;
+    }
+  }
+
+  if (!write) return;
+  T* dst = reinterpret_cast<T*>(p.state) + out_slot * p.ssl + c0 * p.ssd;
+  // The whole line is rewritten: through LDS too (every lane's own part).
+  const bool whole = stage && run == p.S && kept == keep && in_ok;
+  T* line = dst;
+  if (whole) dst = own;
+#pragma unroll
+  for (int i = 0; i < kShortKeep; ++i)
+    if (i < kept)
+#pragma unroll
+      for (int u = 0; u < VEC; ++u) dst[u * p.ssd + i * p.sss] = old[i][u];
+  // Entries past the loaded ones; reads run ahead of the writes (from >= 1).
+  for (int64_t i = kShortKeep; i < kept; ++i)
+#pragma unroll
+    for (int u = 0; u < VEC; ++u) dst[u * p.ssd + i * p.sss] = src[u * p.ssd + (from + i) * p.sss];
+  for (int64_t i = keep; i < run; ++i) {
+    const VT xv = *reinterpret_cast<const VT*>(x + (len - run + i) * p.sx);
+#pragma unroll
+    for (int u = 0; u < VEC; ++u) dst[u * p.ssd + i * p.sss] = xv.v[u];
+  }
+  if (whole) {
+    __syncthreads();
+    u32x4* g = reinterpret_cast<u32x4*>(line - threadIdx.x * VEC * p.S);
+    for (int i = threadIdx.x; i < nvec; i += 256) g[i] = reinterpret_cast<const u32x4*>(short_lds)[i];
+  }
+}
+
+template <typename T, int VEC>
+int launch_short_w(VarlenParams p, hipStream_t s) {
+  p.ncb = cdiv(p.D, 256 * VEC);
+  if (p.ncb * p.B > INT32_MAX) return XK_ERR_UNSUPPORTED;
+  const int64_t bytes = 256 * VEC * p.S * static_cast<int64_t>(sizeof(T));
+  p.short_stage = p.sss == 1 && p.ssd == p.S && p.ssl * static_cast<int64_t>(sizeof(T)) % 16 == 0 &&
+                  aligned(p.state, 16) && bytes <= kShortLds;
+  const uint32_t lds = p.short_stage ? static_cast<uint32_t>(bytes) : 0;
+  const dim3 grid(static_cast<uint32_t>(p.ncb * p.B));
+  switch (p.W) {
+#define XK_W(n) \
+  case n:                                                                       \
+    if (p.silu_on)                                                              \
+      hipLaunchKernelGGL((conv1d_short_kernel<T, n, VEC, true>), grid, dim3(256), lds, s, p); \
+    else                                                                        \
+      hipLaunchKernelGGL((conv1d_short_kernel<T, n, VEC, false>), grid, dim3(256), lds, s, p); \
+    break;
+    XK_W(1) XK_W(2) XK_W(3) XK_W(4) XK_W(5) XK_W(6) XK_W(7) XK_W(8)
+#undef XK_W
+    default: return XK_ERR_UNSUPPORTED;
+  }
+  return launch_status();
+}
+
 template <typename T, int VEC>
 int launch_varlen_w(VarlenParams p, hipStream_t s) {
   p.ncb = cdiv(p.D, 256 * VEC);
@@ -543,6 +711,12 @@ int launch_varlen(VarlenParams p, xk_dtype dt, hipStream_t s) {
   const bool vec = p.D % kV == 0 && p.sx % kV == 0 && p.so % kV == 0 &&
                    aligned(p.x, 16) && aligned(p.out, 16);
   p.w_vec = p.wdt == dt && p.swd == p.W && p.sww == 1 && aligned(p.w, 16);
+  if (p.max_query_len <= kShortLen && p.num_tokens <= kShortLen * p.B &&
+      cdiv(p.D, 256) * p.B <= INT32_MAX) {
+    const bool pair = p.D % 2 == 0 && p.sx % 2 == 0 && p.so % 2 == 0 &&
+                      aligned(p.x, 2 * sizeof(T)) && aligned(p.out, 2 * sizeof(T));
+    return pair ? launch_short_w<T, 2>(p, s) : launch_short_w<T, 1>(p, s);
+  }
   return vec ? launch_varlen_w<T, kV>(p, s) : launch_varlen_w<T, 1>(p, s);
 }
 
