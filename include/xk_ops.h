@@ -219,6 +219,20 @@ int xk_gdn_recurrent(
     int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V, float scale,
     int use_qk_l2norm, int inplace_final_state, void* stream);
 
+/* xk_gdn_recurrent with q, k and v as views of wider rows (the conv's
+ * output): the pitch between tokens in elements, heads dense within a token
+ * (at least H * K, H * K and HV * V, else XK_ERR_INVALID). */
+int xk_gdn_recurrent_strided(
+    const void* q, int64_t stride_q_tok, const void* k, int64_t stride_k_tok, const void* v,
+    int64_t stride_v_tok, xk_dtype dtype, const void* g,
+    xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
+    const float* initial_state, int64_t stride_h0_slot, float* final_state,
+    int64_t stride_ht_slot, int64_t num_slots, const void* cu_seqlens,
+    xk_dtype cu_dtype, const int32_t* ssm_state_indices, int64_t stride_idx_seq,
+    int64_t stride_idx_tok, const int32_t* num_accepted_tokens, int64_t N,
+    int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V, float scale,
+    int use_qk_l2norm, int inplace_final_state, void* stream);
+
 /* ------------------------------------------------------------------------
  * GDN gating (the step before both gated-delta-rule forms).
  * Replaces xllm::kernel::npu::npu_fused_gdn_gating
@@ -355,6 +369,19 @@ int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                      int64_t HV);
 int xk_gdn_chunk_fwd(
     const void* q, const void* k, const void* v, xk_dtype dtype, const void* g,
+    xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
+    const float* initial_state, float* final_state, const void* cu_seqlens,
+    xk_dtype cu_dtype, int64_t N, int64_t total_tokens, int64_t H, int64_t HV,
+    int64_t K, int64_t V, float scale, int use_qk_l2norm, void* workspace,
+    size_t workspace_bytes, void* stream);
+
+/* xk_gdn_chunk_fwd with q / k and v as views of wider rows (the conv's
+ * output): the pitch between tokens in elements, shared by q and k, heads
+ * dense within a token (at least H * K and HV * V and multiples of 8, else
+ * XK_ERR_INVALID). */
+int xk_gdn_chunk_fwd_strided(
+    const void* q, const void* k, int64_t stride_qk_tok, const void* v, int64_t stride_v_tok,
+    xk_dtype dtype, const void* g,
     xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
     const float* initial_state, float* final_state, const void* cu_seqlens,
     xk_dtype cu_dtype, int64_t N, int64_t total_tokens, int64_t H, int64_t HV,

@@ -54,6 +54,9 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "xk_gdn_recurrent": (
         [P, P, P, INT, P, INT, P, INT, P, P, I64, P, I64, I64, P, INT, P, I64,
          I64, P, I64, I64, I64, I64, I64, I64, F32, INT, INT, P], INT),
+    "xk_gdn_recurrent_strided": (
+        [P, I64, P, I64, P, I64, INT, P, INT, P, INT, P, P, I64, P, I64, I64, P, INT, P, I64,
+         I64, P, I64, I64, I64, I64, I64, I64, F32, INT, INT, P], INT),
     "xk_fused_gdn_gating": ([P, P, P, P, P, P, I64, I64, F32, F32, INT, P], INT),
     "xk_gdn_sigmoid_gating_update": (
         [P, P, P, F32, F32, P, P, P, P, INT, P, P, I64, I64, P, P, I64, I64, I64,
@@ -71,6 +74,9 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "xk_gdn_chunk_workspace_bytes": ([I64, I64, I64], I64),
     "xk_gdn_chunk_fwd": (
         [P, P, P, INT, P, INT, P, INT, P, P, P, P, INT, I64, I64, I64, I64, I64,
+         I64, F32, INT, P, SZ, P], INT),
+    "xk_gdn_chunk_fwd_strided": (
+        [P, P, I64, P, I64, INT, P, INT, P, INT, P, P, P, P, INT, I64, I64, I64, I64, I64,
          I64, F32, INT, P, SZ, P], INT),
     "xk_gdn_chunk_fwd_noalloc": (
         [P, P, P, INT, P, INT, P, INT, P, P, P, P, INT, I64, I64, I64, I64, I64,

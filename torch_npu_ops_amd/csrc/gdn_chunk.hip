@@ -80,9 +80,10 @@ __device__ __forceinline__ int img_index(int w, int kk) { return w < 2 ? w : 2 *
 constexpr int kDump = kC * kBVMax * 2;
 
 struct ChunkParams {
-  const void* q;  // [T, H, K]
+  const void* q;  // [T, H, K], token pitch sqk
   const void* k;
-  const void* v;  // [T, HV, V]
+  const void* v;  // [T, HV, V], token pitch sv
+  uint32_t sqk, sv;  // elements; views of a wider row (the conv's output) are read in place
   const void* g;  // [T, HV]
   const void* beta;
   void* o;  // [T, HV, V]
@@ -279,7 +280,7 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   float* rqv = vec[wid][3];
   const int hq = hv / (p.HV / p.H);
   constexpr int KK = K / 32;
-  const int64_t rs = static_cast<int64_t>(p.H) * K;
+  const int64_t rs = p.sqk;
 
   // K rows of the chunk as MFMA operands (A and B^T read the same rows),
   // loaded quad-contiguously (q4_load; rows >= L repeat row L-1).  Every
@@ -467,19 +468,19 @@ struct OutOps {          // consumed by the output o = cq (Q S) + Aq Vn
 template <int K, int BV>
 __device__ __forceinline__ void load_early(const ChunkParams& p, EarlyOps<K / 32, BV / 32>& ops,
                                            int64_t s, int L, int64_t cidx, int hv, int hq,
-                                           uint32_t vrow, int vcol0) {
+                                           int vcol0) {
   const int lane = threadIdx.x & 63, wid = wave_index();
   const int l15 = lane & 15, lg = lane >> 4;
-  const uint32_t rs = static_cast<uint32_t>(p.H) * K;
+  const uint32_t rs = p.sqk;
   const WaveRows wr = wave_rows(s, L, wid);
   const char* kb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.k) +
                                                  wr.row0 * rs + hq * K);
   q4_load_b(kb, 2 * rs, wr.lw, ops.kA);
   const char* vb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.v) +
-                                                 wr.row0 * vrow + vcol0);
+                                                 wr.row0 * p.sv + vcol0);
 #pragma unroll
   for (int j = 0; j < BV / 32; ++j)
-    ops.vA[j] = *reinterpret_cast<const bf8_t*>(vb + row_off(l15, wr.lw, 2 * vrow, 32 * j + 8 * lg));
+    ops.vA[j] = *reinterpret_cast<const bf8_t*>(vb + row_off(l15, wr.lw, 2 * p.sv, 32 * j + 8 * lg));
   const float* sc = reinterpret_cast<const float*>(rec_at(p, cidx, hv) + 3 * kMat);
   const int r4 = wid * 16 + 4 * lg;
   ops.ck = *reinterpret_cast<const f4_t*>(sc + 1 * kC + r4);
@@ -510,7 +511,7 @@ __device__ __forceinline__ void load_out(const ChunkParams& p, OutOps<K / 32>& o
                                          int L, int64_t cidx, int hv, int hq) {
   const int lane = threadIdx.x & 63, wid = wave_index();
   const int l15 = lane & 15;
-  const uint32_t rs = static_cast<uint32_t>(p.H) * K;
+  const uint32_t rs = p.sqk;
   const WaveRows wr = wave_rows(s, L, wid);
   const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.q) +
                                                  wr.row0 * rs + hq * K);
@@ -580,7 +581,7 @@ gdn_chunk_state_kernel(ChunkParams p, int nvt) {
       }
   };
   publish_state();
-  const uint32_t vrow = static_cast<uint32_t>(p.HV) * V;  // v / o token stride
+  const uint32_t vrow = static_cast<uint32_t>(p.HV) * V;  // o token stride
   const int vcol0 = hv * V + v0;
   const bf8_t sel[2] = {select_op(0), select_op(1)};
   EarlyOps<KK, BV / 32> opsA, opsB;
@@ -588,7 +589,7 @@ gdn_chunk_state_kernel(ChunkParams p, int nvt) {
   OutOps<KK> outo;
   if (nch > 0) {
     const int L0 = static_cast<int>(min<int64_t>(kC, eos - bos));
-    load_early<K, BV>(p, opsA, bos, L0, cidx0, hv, hq, vrow, vcol0);
+    load_early<K, BV>(p, opsA, bos, L0, cidx0, hv, hq, vcol0);
     // Keep the early group ahead of the others, in loop order: the loop's
     // wait counts are fixed by the shortest distance (in memory operations)
     // between a load and its first use over every path, this one included,
@@ -613,7 +614,7 @@ gdn_chunk_state_kernel(ChunkParams p, int nvt) {
     const int64_t cn = min(ci + 1, nch - 1);
     const int64_t sn = bos + cn * kC;
     const int Ln = static_cast<int>(min<int64_t>(kC, eos - sn));
-    load_early<K, BV>(p, nxt, sn, Ln, cidx0 + cn, hv, hq, vrow, vcol0);
+    load_early<K, BV>(p, nxt, sn, Ln, cidx0 + cn, hv, hq, vcol0);
 
     // KS = K S (hi/lo S): rows wid*16.., columns nj*16..; K's rows come
     // from the chunk's key tile.
@@ -936,12 +937,12 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   publish_state();
   const uint32_t vrow = static_cast<uint32_t>(p.HV) * V;
   const int vcol0 = hv * V + v0 + cb;
-  const uint32_t rb = static_cast<uint32_t>(p.H) * K * 2;  // q / k row bytes
+  const uint32_t rb = p.sqk * 2;  // q / k row pitch in bytes
   const bf8_t sel[2] = {select_op(0), select_op(1)};
 
   auto load_early8 = [&](EarlyOps8& o, int64_t s, int L, int64_t cidx) {
-    const char* kb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.k) + s * p.H * K + hq * K);
-    const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.q) + s * p.H * K + hq * K);
+    const char* kb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.k) + s * p.sqk + hq * K);
+    const char* qb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.q) + s * p.sqk + hq * K);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const uint32_t off = static_cast<uint32_t>(min(wr * 16 + cg * 8 + 4 * j + rl, L - 1)) * rb + 16u * ch;
@@ -950,8 +951,8 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     }
     const WaveRows wrs = wave_rows(s, L, wr);
     const char* vb = reinterpret_cast<const char*>(reinterpret_cast<const bf16*>(p.v) +
-                                                   wrs.row0 * vrow + vcol0);
-    o.vA = *reinterpret_cast<const bf8_t*>(vb + row_off(l15, wrs.lw, 2 * vrow, 8 * lg));
+                                                   wrs.row0 * p.sv + vcol0);
+    o.vA = *reinterpret_cast<const bf8_t*>(vb + row_off(l15, wrs.lw, 2 * p.sv, 8 * lg));
     if (is_m) o.vA = bf8_t{};  // a transition has no values (and takes no NaN from them)
     // The factor block (cq, ck, beta, ed: 1 KB) in one load per wave; the
     // wave-uniform e^{g_last} through the scalar cache.
@@ -1417,7 +1418,7 @@ int chunk_args_status(const void* q, const void* k, const void* v, xk_dtype dtyp
                       const void* g, xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype,
                       const void* o, const void* cu_seqlens, xk_dtype cu_dtype, int64_t N,
                       int64_t total_tokens, int64_t H, int64_t HV, int64_t K, int64_t V,
-                      bool* empty) {
+                      int64_t sqk, int64_t sv, bool* empty) {
   *empty = false;
   if (N < 0 || total_tokens < 0 || H <= 0 || HV <= 0 || HV % H != 0)
     return XK_ERR_INVALID;
@@ -1428,8 +1429,11 @@ int chunk_args_status(const void* q, const void* k, const void* v, xk_dtype dtyp
   if (cu_dtype != XK_I32 && cu_dtype != XK_I64) return XK_ERR_UNSUPPORTED;
   if (K != 128 || V % 32 != 0 || V <= 0) return XK_ERR_UNSUPPORTED;
   // Row pitches of q / k and v / o in bytes feed 24-bit multiplies.
-  if (H * K * 2 >= (int64_t{1} << 24) || HV * V * 2 >= (int64_t{1} << 24))
+  if (H * K * 2 >= (int64_t{1} << 24) || HV * V * 2 >= (int64_t{1} << 24) ||
+      sqk * 2 >= (int64_t{1} << 24) || sv * 2 >= (int64_t{1} << 24))
     return XK_ERR_UNSUPPORTED;
+  // Rows must not overlap and start at 16-byte boundaries.
+  if (sqk < H * K || sv < HV * V || sqk % 8 != 0 || sv % 8 != 0) return XK_ERR_INVALID;
   if (N == 0 || total_tokens == 0) {
     *empty = true;
     return XK_OK;
@@ -1445,16 +1449,17 @@ int chunk_args_status(const void* q, const void* k, const void* v, xk_dtype dtyp
 }  // namespace
 }  // namespace xk
 
-extern "C" int xk_gdn_chunk_fwd(
-    const void* q, const void* k, const void* v, xk_dtype dtype, const void* g,
-    xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
+extern "C" int xk_gdn_chunk_fwd_strided(
+    const void* q, const void* k, int64_t stride_qk_tok, const void* v, int64_t stride_v_tok,
+    xk_dtype dtype, const void* g, xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
     const float* initial_state, float* final_state, const void* cu_seqlens,
     xk_dtype cu_dtype, int64_t N, int64_t total_tokens, int64_t H, int64_t HV,
     int64_t K, int64_t V, float scale, int use_qk_l2norm, void* workspace,
     size_t workspace_bytes, void* stream) {
   bool empty = false;
-  const int ast = chunk_args_status(q, k, v, dtype, g, g_dtype, beta, beta_dtype, o, cu_seqlens,
-                                    cu_dtype, N, total_tokens, H, HV, K, V, &empty);
+  const int ast =
+      chunk_args_status(q, k, v, dtype, g, g_dtype, beta, beta_dtype, o, cu_seqlens, cu_dtype, N,
+                        total_tokens, H, HV, K, V, stride_qk_tok, stride_v_tok, &empty);
   if (ast != XK_OK || empty) return ast;
   const int64_t need = least_workspace(total_tokens, N, HV);
   if (!workspace || static_cast<int64_t>(workspace_bytes) < need) return XK_ERR_WORKSPACE;
@@ -1463,6 +1468,8 @@ extern "C" int xk_gdn_chunk_fwd(
   p.q = q;
   p.k = k;
   p.v = v;
+  p.sqk = static_cast<uint32_t>(stride_qk_tok);
+  p.sv = static_cast<uint32_t>(stride_v_tok);
   p.g = g;
   p.beta = beta;
   p.o = o;
@@ -1504,6 +1511,19 @@ extern "C" int xk_gdn_chunk_fwd(
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (g_dtype == XK_F32) return chunk_beta<128, float>(p, V, beta_dtype, s);
   return chunk_beta<128, bf16>(p, V, beta_dtype, s);
+}
+
+extern "C" int xk_gdn_chunk_fwd(
+    const void* q, const void* k, const void* v, xk_dtype dtype, const void* g,
+    xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
+    const float* initial_state, float* final_state, const void* cu_seqlens,
+    xk_dtype cu_dtype, int64_t N, int64_t total_tokens, int64_t H, int64_t HV,
+    int64_t K, int64_t V, float scale, int use_qk_l2norm, void* workspace,
+    size_t workspace_bytes, void* stream) {
+  return xk_gdn_chunk_fwd_strided(q, k, H * K, v, HV * V, dtype, g, g_dtype, beta, beta_dtype, o,
+                                  initial_state, final_state, cu_seqlens, cu_dtype, N,
+                                  total_tokens, H, HV, K, V, scale, use_qk_l2norm, workspace,
+                                  workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1562,7 +1582,7 @@ extern "C" int xk_gdn_chunk_fwd_noalloc(
   // The same argument checks as xk_gdn_chunk_fwd, before the size check.
   bool empty = false;
   const int ast = chunk_args_status(q, k, v, dtype, g, g_dtype, beta, beta_dtype, o, cu_seqlens,
-                                    cu_dtype, N, total_tokens, H, HV, K, V, &empty);
+                                    cu_dtype, N, total_tokens, H, HV, K, V, H * K, HV * V, &empty);
   if (ast != XK_OK || empty) return ast;
   const int64_t need = least_workspace(total_tokens, N, HV);
   if (need > kNoAllocScratchBytes) return XK_ERR_SCRATCH;

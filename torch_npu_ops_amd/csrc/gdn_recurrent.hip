@@ -285,6 +285,7 @@ struct RecParams {
   const void* q;
   const void* k;
   const void* v;
+  int64_t sq, sk, sv;  // token pitches of q, k, v (elements); heads dense within a token
   const void* g;
   const void* beta;
   void* o;
@@ -350,9 +351,9 @@ __global__ void __launch_bounds__(kThreads) gdn_recurrent_kernel(RecParams p) {
   };
   auto load_in = [&](int64_t tok) {
     TokIn r;
-    r.q = tid < K ? ldf<T>(p.q, (tok * p.H + hq) * K + tid) : 0.f;
-    r.k = tid < K ? ldf<T>(p.k, (tok * p.H + hq) * K + tid) : 0.f;
-    r.v = tid < VT ? ldf<T>(p.v, (tok * p.HV + hv) * V + cs * VT + tid) : 0.f;
+    r.q = tid < K ? ldf<T>(p.q, tok * p.sq + hq * K + tid) : 0.f;
+    r.k = tid < K ? ldf<T>(p.k, tok * p.sk + hq * K + tid) : 0.f;
+    r.v = tid < VT ? ldf<T>(p.v, tok * p.sv + hv * V + cs * VT + tid) : 0.f;
     r.g = ldf<GT>(p.g, tok * p.HV + hv);
     r.b = p.beta ? ldf<BT>(p.beta, tok * p.HV + hv) : 1.0f;
     if (p.gating) {
@@ -681,8 +682,9 @@ int fused_g(const FusedParams& p, xk_dtype gdt, xk_dtype bdt, hipStream_t s) {
 
 using namespace xk;
 
-extern "C" int xk_gdn_recurrent(
-    const void* q, const void* k, const void* v, xk_dtype dtype, const void* g,
+extern "C" int xk_gdn_recurrent_strided(
+    const void* q, int64_t stride_q_tok, const void* k, int64_t stride_k_tok, const void* v,
+    int64_t stride_v_tok, xk_dtype dtype, const void* g,
     xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
     const float* initial_state, int64_t stride_h0_slot, float* final_state,
     int64_t stride_ht_slot, int64_t num_slots, const void* cu_seqlens,
@@ -691,6 +693,7 @@ extern "C" int xk_gdn_recurrent(
     int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V, float scale,
     int use_qk_l2norm, int inplace_final_state, void* stream) {
   if (N < 0 || T < 0 || H <= 0 || HV <= 0 || HV % H != 0) return XK_ERR_INVALID;
+  if (stride_q_tok < H * K || stride_k_tok < H * K || stride_v_tok < HV * V) return XK_ERR_INVALID;
   if (!is_float_dtype(dtype) || !is_float_dtype(g_dtype) ||
       (beta && !is_float_dtype(beta_dtype)))
     return XK_ERR_UNSUPPORTED;
@@ -707,6 +710,9 @@ extern "C" int xk_gdn_recurrent(
   p.q = q;
   p.k = k;
   p.v = v;
+  p.sq = stride_q_tok;
+  p.sk = stride_k_tok;
+  p.sv = stride_v_tok;
   p.g = g;
   p.beta = beta;
   p.o = o;
@@ -735,6 +741,23 @@ extern "C" int xk_gdn_recurrent(
   if (K == 128 && V == 64) return rec_t<128, 64>(p, dtype, g_dtype, bdt, s);
   if (K == 64 && V == 128) return rec_t<64, 128>(p, dtype, g_dtype, bdt, s);
   return XK_ERR_UNSUPPORTED;
+}
+
+extern "C" int xk_gdn_recurrent(
+    const void* q, const void* k, const void* v, xk_dtype dtype, const void* g,
+    xk_dtype g_dtype, const void* beta, xk_dtype beta_dtype, void* o,
+    const float* initial_state, int64_t stride_h0_slot, float* final_state,
+    int64_t stride_ht_slot, int64_t num_slots, const void* cu_seqlens,
+    xk_dtype cu_dtype, const int32_t* ssm_state_indices, int64_t stride_idx_seq,
+    int64_t stride_idx_tok, const int32_t* num_accepted_tokens, int64_t N,
+    int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V, float scale,
+    int use_qk_l2norm, int inplace_final_state, void* stream) {
+  return xk_gdn_recurrent_strided(q, H * K, k, H * K, v, HV * V, dtype, g, g_dtype, beta,
+                                  beta_dtype, o, initial_state, stride_h0_slot, final_state,
+                                  stride_ht_slot, num_slots, cu_seqlens, cu_dtype,
+                                  ssm_state_indices, stride_idx_seq, stride_idx_tok,
+                                  num_accepted_tokens, N, T, H, HV, K, V, scale, use_qk_l2norm,
+                                  inplace_final_state, stream);
 }
 
 namespace {
@@ -908,6 +931,8 @@ extern "C" int xk_gdn_sigmoid_gating_update(
   p.q = q;
   p.k = k;
   p.v = v;
+  p.sq = p.sk = H * K;
+  p.sv = HV * V;
   p.g = a;
   p.beta = b;
   p.o = o;

@@ -84,6 +84,23 @@ torch::Tensor workspace(int64_t bytes, const torch::Device& dev) {
                       torch::TensorOptions().dtype(torch::kUInt8).device(dev));
 }
 
+// x [B, T, heads, d] with the B * T token rows one pitch apart and each row's
+// heads dense: itself when it already is (a slice of a wider row, such as
+// the conv's output, needs no copy), else a contiguous copy.  `align`: the
+// elements that pitch and start have to be a multiple of.
+torch::Tensor token_rows(const torch::Tensor& x, int64_t align) {
+  const int64_t row = x.size(2) * x.size(3), pitch = x.stride(1);
+  const bool ok = x.numel() > 0 && (x.size(3) == 1 || x.stride(3) == 1) &&
+                  (x.size(2) == 1 || x.stride(2) == x.size(3)) && pitch >= row &&
+                  pitch % align == 0 && pitch * 2 < (int64_t{1} << 24) &&
+                  (x.size(0) == 1 || x.stride(0) == x.size(1) * pitch) &&
+                  reinterpret_cast<uintptr_t>(x.data_ptr()) % (align * x.element_size()) == 0;
+  return ok ? x : x.contiguous();
+}
+int64_t token_pitch(const torch::Tensor& x) {
+  return x.is_contiguous() ? x.size(2) * x.size(3) : x.stride(1);
+}
+
 torch::Tensor layer_norm_impl(const torch::Tensor& x, const torch::Tensor& weight,
                               const torch::Tensor& bias, double eps,
                               const std::optional<torch::Tensor>& z, int64_t group_size,
@@ -335,7 +352,7 @@ std::pair<torch::Tensor, torch::Tensor> npu_fused_recurrent_gated_delta_rule(
   TORCH_CHECK(has(initial_state), "initial_state must be provided");
   const float sc = scale.has_value() ? *scale : 1.0f / std::sqrt(static_cast<float>(K));
   const int64_t N = has(cu_seqlens) ? cu_seqlens->numel() - 1 : B;
-  auto qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous(), gc = g.contiguous();
+  auto qc = token_rows(q, 1), kc = token_rows(k, 1), vc = token_rows(v, 1), gc = g.contiguous();
   torch::Tensor bc;
   if (has(beta)) bc = beta->contiguous();
   auto o = torch::empty({B, T, HV, V}, q.options());
@@ -354,14 +371,14 @@ std::pair<torch::Tensor, torch::Tensor> npu_fused_recurrent_gated_delta_rule(
   }
   if (has(num_accepted_tokens)) acc = num_accepted_tokens->to(torch::kInt32).contiguous();
   if (has(cu_seqlens)) cu = cu_seqlens->contiguous();
-  check(xk_gdn_recurrent(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), xdt(qc), gc.data_ptr(),
-                         xdt(gc), ptr(bc), bc.defined() ? xdt(bc) : XK_F32, o.data_ptr(),
-                         static_cast<const float*>(h0.data_ptr()), h0.stride(0),
-                         static_cast<float*>(fin.data_ptr()), fin.stride(0), h0.size(0), ptr(cu),
-                         cu.defined() ? xdt(cu) : XK_I32,
-                         static_cast<const int32_t*>(ptr(idx)), s0, s1,
-                         static_cast<const int32_t*>(ptr(acc)), N, cu.defined() ? 0 : T, H, HV,
-                         K, V, sc, /*use_qk_l2norm=*/1, inplace_final_state, stream_of(q)),
+  check(xk_gdn_recurrent_strided(
+            qc.data_ptr(), token_pitch(qc), kc.data_ptr(), token_pitch(kc), vc.data_ptr(),
+            token_pitch(vc), xdt(qc), gc.data_ptr(), xdt(gc), ptr(bc),
+            bc.defined() ? xdt(bc) : XK_F32, o.data_ptr(), static_cast<const float*>(h0.data_ptr()),
+            h0.stride(0), static_cast<float*>(fin.data_ptr()), fin.stride(0), h0.size(0), ptr(cu),
+            cu.defined() ? xdt(cu) : XK_I32, static_cast<const int32_t*>(ptr(idx)), s0, s1,
+            static_cast<const int32_t*>(ptr(acc)), N, cu.defined() ? 0 : T, H, HV, K, V, sc,
+            /*use_qk_l2norm=*/1, inplace_final_state, stream_of(q)),
         "xk_gdn_recurrent");
   return {o, fin};
 }
@@ -545,7 +562,8 @@ std::pair<torch::Tensor, torch::Tensor> npu_chunk_gated_delta_rule(
               "g must have shape [B, T, H].");
   auto [cu, N] = seqs(B, T, cu_seqlens, q.device());
   const float sc = scale.has_value() ? *scale : std::pow(static_cast<float>(K), -0.5f);
-  auto qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
+  auto qc = token_rows(q, 8), kc = token_rows(k, 8), vc = token_rows(v, 8);
+  if (token_pitch(qc) != token_pitch(kc)) qc = q.contiguous(), kc = k.contiguous();
   auto gc = g.contiguous(), bc = beta.contiguous();
   torch::Tensor h0;
   if (has(initial_state)) h0 = initial_state->to(torch::kFloat32).contiguous();
@@ -553,11 +571,12 @@ std::pair<torch::Tensor, torch::Tensor> npu_chunk_gated_delta_rule(
   torch::Tensor fin = output_final_state ? torch::empty({N, HV, K, V}, f32) : torch::Tensor();
   auto o = torch::empty({B, T, HV, V}, q.options());
   auto ws = workspace(xk_gdn_chunk_workspace_bytes(B * T, N, HV), q.device());
-  check(xk_gdn_chunk_fwd(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), xdt(qc), gc.data_ptr(),
-                         xdt(gc), bc.data_ptr(), xdt(bc), o.data_ptr(),
-                         static_cast<const float*>(ptr(h0)), static_cast<float*>(mptr(fin)),
-                         cu.data_ptr(), xdt(cu), N, B * T, H, HV, K, V, sc,
-                         use_qk_l2norm_in_kernel, ws.data_ptr(), ws.numel(), stream_of(q)),
+  check(xk_gdn_chunk_fwd_strided(
+            qc.data_ptr(), kc.data_ptr(), token_pitch(qc), vc.data_ptr(), token_pitch(vc), xdt(qc),
+            gc.data_ptr(), xdt(gc), bc.data_ptr(), xdt(bc), o.data_ptr(),
+            static_cast<const float*>(ptr(h0)), static_cast<float*>(mptr(fin)), cu.data_ptr(),
+            xdt(cu), N, B * T, H, HV, K, V, sc, use_qk_l2norm_in_kernel, ws.data_ptr(), ws.numel(),
+            stream_of(q)),
         "xk_gdn_chunk_fwd");
   return {o, fin};
 }
