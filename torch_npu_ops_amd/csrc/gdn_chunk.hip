@@ -94,6 +94,10 @@ struct ChunkParams {
   int32_t* chunk_off;  // [N+1] workspace
   int32_t* seq_order;  // [N] workspace: sequences, longest first
   int2* ctab;          // [NTmax] workspace: (first token, length) per chunk
+  // [N], N <= kWaveSeqs, in the place of the three above (which are unused
+  // then): sequence, first global chunk, first and end token of rank r,
+  // longest first.
+  int4* seqtab;
   bf16* dump;          // [64 * kBVMax] workspace: sink for padded-row stores
   char* rec;           // [NTmax, HV] records of kRec bytes, workspace
   int64_t N, NTmax;
@@ -205,6 +209,19 @@ __device__ __forceinline__ WaveSegs wave_segs(const ChunkParams& p) {
   return w;
 }
 
+// Sequence of rank r (wave-uniform).
+struct SeqEntry {
+  int64_t n, c0, bos, eos;
+};
+__device__ __forceinline__ SeqEntry ranked_seq(const ChunkParams& p, int64_t r) {
+  if (p.N <= kWaveSeqs) {
+    const int4 e = p.seqtab[r];
+    return {e.x, e.y, e.z, e.w};
+  }
+  const int64_t n = p.seq_order[r];
+  return {n, p.chunk_off[n], cu_at(p, n), cu_at(p, n + 1)};
+}
+
 // Rows >= L of the K / Q operands (q4_load) repeat row L-1; here every
 // consumer zeroes them through factors that are 0 there (beta, ck, ed, the
 // masks of M and Aq).
@@ -256,9 +273,23 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   const int hg4 = (p.HV + 3) >> 2;
   const int64_t c = blockIdx.x / hg4;
   const int hv = static_cast<int>(blockIdx.x % hg4) * 4 + wid;
-  if (c == p.NTmax) {  // the one block past the chunks (launched with seg_max)
-    const int len = wave_seg_len(p);
-    if (threadIdx.x == 0) *p.seg_len = len;
+  if (c == p.NTmax) {
+    // The one block past the chunks (N <= kWaveSeqs): the sequences by rank,
+    // which the state kernel's blocks would otherwise each work out (a loop
+    // over N in every wave), and the segment plan.
+    if (wid > 0) return;
+    const WaveSeqs w = wave_seqs(p);
+    int rank = 0;
+    for (int m = 0; m < static_cast<int>(p.N); ++m) {
+      const int32_t cm = __builtin_amdgcn_readlane(w.cnt, m);
+      rank += (cm > w.cnt) || (cm == w.cnt && m < lane);
+    }
+    if (lane < p.N)
+      p.seqtab[rank] = make_int4(lane, w.incl - w.cnt, static_cast<int>(w.a), static_cast<int>(w.b));
+    if (p.seg_max) {
+      const int len = wave_seg_len(p);
+      if (lane == 0) *p.seg_len = len;
+    }
     return;
   }
   int64_t s;
@@ -544,13 +575,12 @@ gdn_chunk_state_kernel(ChunkParams p, int nvt) {
   const int vt = static_cast<int>(r % nvt);
   const int64_t item = (r / nvt) * 8 + xcd;  // (sequence rank, head) index
   if (item >= p.N * p.HV) return;            // whole block
-  int64_t n, cidx0;
-  find_ranked_seq(p, item / p.HV, n, cidx0);
+  const SeqEntry se = ranked_seq(p, item / p.HV);
+  const int64_t n = se.n, cidx0 = se.c0, bos = se.bos, eos = se.eos;
   const int hv = state_head(static_cast<int>(item % p.HV), p.HV, p.H);
   const int hq = hv / (p.HV / p.H);
   const int V = nvt * BV;
   const int v0 = vt * BV;
-  const int64_t bos = cu_at(p, n), eos = cu_at(p, n + 1);
   // Chunks of this sequence; the NTmax bound keeps a malformed cu_seqlens
   // (never a well-formed one) from reading past the workspace.
   const int64_t nch = max<int64_t>(0, min<int64_t>((eos - bos + kC - 1) / kC, p.NTmax - cidx0));
@@ -860,9 +890,11 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   int before = 0;  // segments of the sequence before this one
   if constexpr (MODE == kSegNone) {
     if (item >= p.N * p.HV) return;
-    find_ranked_seq(p, item / p.HV, n, cidx0);
-    bos = cu_at(p, n);
-    eos = cu_at(p, n + 1);
+    const SeqEntry se = ranked_seq(p, item / p.HV);
+    n = se.n;
+    cidx0 = se.c0;
+    bos = se.bos;
+    eos = se.eos;
     nch = (eos - bos + kC - 1) / kC;
     const int64_t at = (n * p.HV + hv) * K * V;
     s_in = p.h0 ? p.h0 + at : nullptr;
@@ -910,31 +942,6 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   const int scol = is_m ? (vt - nvt) * BV : vt * BV;  // first column of the state block
 
   constexpr int M2 = K / 64;
-  f4_t sreg[M2][NJ];
-#pragma unroll
-  for (int m2 = 0; m2 < M2; ++m2)
-#pragma unroll
-    for (int nj = 0; nj < NJ; ++nj)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kr = wr * (K / 4) + m2 * 16 + 4 * lg + i;
-        const int col = scol + cb + nj * 16 + l15;
-        if (is_m) sreg[m2][nj][i] = kr == col ? 1.f : 0.f;
-        else sreg[m2][nj][i] = s_in ? s_in[static_cast<int64_t>(kr) * V + col] : 0.f;
-      }
-  auto publish_state = [&]() {
-#pragma unroll
-    for (int m2 = 0; m2 < M2; ++m2)
-#pragma unroll
-      for (int nj = 0; nj < NJ; ++nj) {
-        Vec<__bf16, 4> h, l;
-        split4(sreg[m2][nj], h, l);
-        const int k0 = wr * (K / 4) + m2 * 16 + 4 * lg;
-        *reinterpret_cast<Vec<__bf16, 4>*>(&sm.sb[0][sb8_off(cb + nj * 16 + l15, k0)]) = h;
-        *reinterpret_cast<Vec<__bf16, 4>*>(&sm.sb[1][sb8_off(cb + nj * 16 + l15, k0)]) = l;
-      }
-  };
-  publish_state();
   const uint32_t vrow = static_cast<uint32_t>(p.HV) * V;
   const int vcol0 = hv * V + v0 + cb;
   const uint32_t rb = p.sqk * 2;  // q / k row pitch in bytes
@@ -986,6 +993,8 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
   EarlyOps8 opsA, opsB;
   InvOps8 inv;
   OutOps8 outo;
+  // The first chunk's operands are requested before the initial state, so
+  // that a block of a few chunks waits once.
   if (nch > 0) {
     const int L0 = static_cast<int>(min<int64_t>(kC, eos - bos));
     load_early8(opsA, bos, L0, cidx0);
@@ -993,6 +1002,34 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     load_inv8(inv, cidx0);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (kOut) load_out8(outo, cidx0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  f4_t sreg[M2][NJ];
+#pragma unroll
+  for (int m2 = 0; m2 < M2; ++m2)
+#pragma unroll
+    for (int nj = 0; nj < NJ; ++nj)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int kr = wr * (K / 4) + m2 * 16 + 4 * lg + i;
+        const int col = scol + cb + nj * 16 + l15;
+        if (is_m) sreg[m2][nj][i] = kr == col ? 1.f : 0.f;
+        else sreg[m2][nj][i] = s_in ? s_in[static_cast<int64_t>(kr) * V + col] : 0.f;
+      }
+  auto publish_state = [&]() {
+#pragma unroll
+    for (int m2 = 0; m2 < M2; ++m2)
+#pragma unroll
+      for (int nj = 0; nj < NJ; ++nj) {
+        Vec<__bf16, 4> h, l;
+        split4(sreg[m2][nj], h, l);
+        const int k0 = wr * (K / 4) + m2 * 16 + 4 * lg;
+        *reinterpret_cast<Vec<__bf16, 4>*>(&sm.sb[0][sb8_off(cb + nj * 16 + l15, k0)]) = h;
+        *reinterpret_cast<Vec<__bf16, 4>*>(&sm.sb[1][sb8_off(cb + nj * 16 + l15, k0)]) = l;
+      }
+  };
+  publish_state();
+  if (nch > 0) {
     store_rows(sm.kr[0], opsA.kraw);
     if constexpr (kOut) store_rows(sm.qr, opsA.qraw);
     store_fac(sm.fac[0], opsA.fac);
@@ -1302,7 +1339,7 @@ int launch_chunk(const ChunkParams& p, int64_t V, hipStream_t s) {
   const int64_t prep_blocks = p.NTmax * ((p.HV + 3) / 4);
   if (prep_blocks >= INT32_MAX) return XK_ERR_UNSUPPORTED;
   hipLaunchKernelGGL((gdn_chunk_prep_kernel<K, GT, BT>),
-                     dim3(static_cast<uint32_t>(prep_blocks) + (p.seg_max ? 1 : 0)),
+                     dim3(static_cast<uint32_t>(prep_blocks) + (p.N <= kWaveSeqs ? 1 : 0)),
                      dim3(kTh), 0, s, p);
   st = launch_status();
   if (st) return st;
@@ -1478,6 +1515,9 @@ extern "C" int xk_gdn_chunk_fwd_strided(
   p.cu = cu_seqlens;
   p.cu_i64 = cu_dtype == XK_I64;
   char* ws = static_cast<char*>(workspace);
+  // 16 N <= align256(4 (N + 1)) + align256(4 N) + align256(8 N) for every N
+  // up to kWaveSeqs.
+  p.seqtab = reinterpret_cast<int4*>(ws);
   p.chunk_off = reinterpret_cast<int32_t*>(ws);
   ws += align256(4 * (N + 1));
   p.seq_order = reinterpret_cast<int32_t*>(ws);
