@@ -262,7 +262,7 @@ __device__ __forceinline__ void row_scales(const bf8_t (&x)[4][KK], float* r, in
 template <int K, typename GT, typename BT>
 __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   __shared__ __align__(16) float lds[4][kC][kLd];
-  __shared__ float vec[4][4][kC];  // gc, beta, r_k, r_q per wave
+  __shared__ __align__(16) float vec[4][5][kC];  // gc, beta, r_k, r_q, c_k per wave
   // Wave index in a scalar register: the exit below is then a scalar branch,
   // and the DPP transposes (q4_to_a) run with every lane of the wave active.
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -309,6 +309,7 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   float* btv = vec[wid][1];
   float* rkv = vec[wid][2];
   float* rqv = vec[wid][3];
+  float* ckv = vec[wid][4];
   const int hq = hv / (p.HV / p.H);
   constexpr int KK = K / 32;
   const int64_t rs = p.sqk;
@@ -346,6 +347,30 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   row_scales<KK>(kop, rkv, p.l2norm);
   __builtin_amdgcn_wave_barrier();
 
+  // The decay exp(gc_i - gc_j) of the tiles below the diagonal ones is a
+  // product of factors of rows, columns and tiles, each <= 1 for decays <= 1
+  // (an underflow of one underflows the product): with G_t = gc at the end
+  // of 16-token block t - 1, row i of block mi and column j of block nj < mi,
+  //   exp(gc_i - gc_j) = exp(gc_i - G_mi) exp(G_mi - G_{nj+1}) exp(G_{nj+1} - gc_j).
+  // An element then takes two multiplies instead of an exponential and six
+  // VALU instructions.  c_k = r_k exp(G_{nj+1} - gc) is formed once per token.
+  // 24 of an M or Aq tile's 40 elements per lane; XX -> XX us at config 4 on
+  // MI355X.
+  ckv[lane] = rkv[lane] * __expf(gcv[lane | 15] - gv);
+  float tile_decay[3];  // exp(G_mi - G_{nj+1}) of (2, 0), (3, 1), (3, 0)
+  {
+    const float g1 = readlane_f32(gv, 15), g2 = readlane_f32(gv, 31), g3 = readlane_f32(gv, 47);
+    tile_decay[0] = __expf(g2 - g1);
+    tile_decay[1] = __expf(g3 - g2);
+    tile_decay[2] = __expf(g3 - g1);
+  }
+  auto tile_scale = [&](int mi, int nj) {
+    return mi - nj == 1 ? 1.f : tile_decay[mi == 2 ? 0 : nj == 1 ? 1 : 2];
+  };
+  // exp(gc_i - G_mi) of the lane's row of block mi.
+  auto row_decay = [&](int mi, float gr) { return mi ? __expf(gr - readlane_f32(gv, 16 * mi - 1)) : 1.f; };
+  __builtin_amdgcn_wave_barrier();
+
   // M = strict_tril(b_i r_i r_j (k_i . k_j) exp(gc_i - gc_j)) into X (the
   // ten lower 16x16 tiles; the strictly upper ones are never read).  The
   // product K_nj K_mi^T is tile (mi, nj) transposed, so a lane holds row
@@ -354,16 +379,24 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   for (int mi = 0; mi < 4; ++mi) {
     const int row = mi * 16 + l15;
     const float fr = btv[row] * rkv[row], gr = gcv[row];
+    const float fd = fr * row_decay(mi, gr);
 #pragma unroll
     for (int nj = 0; nj <= mi; ++nj) {
       f4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) a = mfma16(kop[nj][kk], kop[mi][kk], a);
       f4_t m;
+      if (nj < mi) {
+        const f4_t ck = *reinterpret_cast<const f4_t*>(ckv + nj * 16 + 4 * lg);
+        const float ft = fd * tile_scale(mi, nj);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int col = nj * 16 + 4 * lg + i;
-        m[i] = row > col ? fr * rkv[col] * a[i] * __expf(gr - gcv[col]) : 0.f;
+        for (int i = 0; i < 4; ++i) m[i] = ft * ck[i] * a[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int col = nj * 16 + 4 * lg + i;
+          m[i] = row > col ? fr * rkv[col] * a[i] * __expf(gr - gcv[col]) : 0.f;
+        }
       }
       *reinterpret_cast<f4_t*>(&X[row][nj * 16 + 4 * lg]) = m;
     }
@@ -412,20 +445,27 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
 #pragma unroll
   for (int mi = 0; mi < 4; ++mi) {
     const int row = mi * 16 + l15;
-    const float fr = p.scale * rqv[row], gr = gcv[row];
+    const float fr = row < L ? p.scale * rqv[row] : 0.f, gr = gcv[row];
+    const float fd = fr * row_decay(mi, gr);
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) {
-      f4_t a = {0.f, 0.f, 0.f, 0.f};
+      f4_t val = {0.f, 0.f, 0.f, 0.f};
       if (nj <= mi) {
+        f4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) a = mfma16(kop[nj][kk], qop[mi][kk], a);
-      }
-      f4_t val;
+        if (nj < mi) {
+          const f4_t ck = *reinterpret_cast<const f4_t*>(ckv + nj * 16 + 4 * lg);
+          const float ft = fd * tile_scale(mi, nj);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int col = nj * 16 + 4 * lg + i;
-        val[i] = nj <= mi && row >= col && row < L ? fr * rkv[col] * a[i] * __expf(gr - gcv[col])
-                                                    : 0.f;
+          for (int i = 0; i < 4; ++i) val[i] = ft * ck[i] * a[i];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int col = nj * 16 + 4 * lg + i;
+            val[i] = row >= col ? fr * rkv[col] * a[i] * __expf(gr - gcv[col]) : 0.f;
+          }
+        }
       }
       *reinterpret_cast<f4_t*>(&X[row][nj * 16 + 4 * lg]) = val;
     }
