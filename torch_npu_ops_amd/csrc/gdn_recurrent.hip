@@ -23,7 +23,10 @@
 // cross-wave LDS reduction (o = (e^g h)^T q + (k.q) v', so the update and
 // the output need no second pass); the rank-1 update is applied in
 // registers and the state is written back once.  State traffic uses
-// non-temporal hints: it is read and written exactly once per call.
+// non-temporal hints: it is read and written exactly once per call.  A token
+// takes one barrier (gdn_token); a decode layer's step for one sequence of 32
+// v-heads, replayed from a graph on MI355X, went from 24.1 to 22.9 us with
+// that (six barriers before), large batches stay at the state stream's rate.
 #include "xk_common.h"
 
 namespace xk {
@@ -48,17 +51,12 @@ struct Tile {
   float h[kPasses][4];
 };
 
-// LDS shared by one block: normalised q/k (fp32), v, the reduction scratch
-// and the per-column results.
-template <int K, int V, int NT = kThreads>
-struct Smem {
-  float q[K];
-  float k[K];
-  float v[V];
-  float red[2][NT / kWave][V];  // per-wave partials of h^T k, h^T q
-  float kh[V];
-  float qh[V];
-  float scal[4];  // k.q, ||q||^2, ||k||^2
+// Per-wave partials of h^T k and h^T q, double-buffered from one token (or
+// head) to the next: written before a token's barrier, read until the next
+// one's.
+template <int V, int NT = kThreads>
+struct Partials {
+  float p[2][2][NT / kWave][V];
 };
 
 template <typename T>
@@ -132,24 +130,71 @@ __device__ __forceinline__ AB sigmoid_to(float x) {
   }
 }
 
-// One token of the recurrence on the register tile.  Inputs (q, k already
-// normalised and q scaled) are in sm.q / sm.k / sm.v.  Writes o[V] through
-// `out` (fp32 values, converted by the caller's store functor).
-template <int K, int V, int NT, typename StoreO>
-__device__ __forceinline__ void gdn_token(Tile<K, V, NT>& t, Smem<K, V, NT>& sm,
-                                          float decay, float beta, StoreO store_o) {
+// Sum over the lanes of a wave that differ in lane bits 4 and 5 (STAGE 16 and
+// 32), by swapping 16-lane rows / wave halves of two copies of the value.
+template <int STAGE>
+__device__ __forceinline__ float swap_sum(float v) {
+  static_assert(STAGE == 16 || STAGE == 32, "row or half");
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  typedef unsigned int u2_t __attribute__((ext_vector_type(2)));
+  u2_t r;
+  if constexpr (STAGE == 16) r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  else r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t x = r[0], y = r[1];  // (a bit cast of a vector element reads element 0)
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+
+// Scalars of one token's q and k (raw, fp32, in LDS): rk = 1 / ||k||, rq =
+// scale / ||q|| (norms with the 1e-6 of the l2norm; 1 without it) and kq =
+// rk rq (k . q).  Every wave forms them for itself, so no barrier is needed
+// between them and their use.
+struct QkScales {
+  float rk, rq, kq;
+};
+template <int K>
+__device__ __forceinline__ QkScales qk_scales(const float* q, const float* k, bool l2norm,
+                                              float scale) {
+  const int lane = threadIdx.x % kWave;
+  float sq = 0.f, sk = 0.f, kq = 0.f;
+#pragma unroll
+  for (int i = lane; i < K; i += kWave) {
+    const float qv = q[i], kv = k[i];
+    sq = fmaf(qv, qv, sq);
+    sk = fmaf(kv, kv, sk);
+    kq = fmaf(qv, kv, kq);
+  }
+  sq = group_sum<kWave>(sq);
+  sk = group_sum<kWave>(sk);
+  kq = group_sum<kWave>(kq);
+  QkScales r;
+  r.rk = l2norm ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f;
+  r.rq = (l2norm ? 1.0f / sqrtf(sq + 1e-6f) : 1.0f) * scale;
+  r.kq = kq * r.rk * r.rq;
+  return r;
+}
+
+// One token of the recurrence on the register tile, with one barrier.  q, k
+// and v (raw, fp32, LDS) were complete at the barrier before; `before` runs
+// ahead of this one's barrier (it may fill the other input buffer) and
+// store_o(column, four outputs) is called by the lanes of the first row.
+// Every lane sums the waves' partials of its own four columns after the
+// barrier and applies the norms of q and k as scalars, where writing
+// normalised q and k, then v', back through LDS took five more barriers.
+template <int K, int V, int NT, typename Before, typename StoreO>
+__device__ __forceinline__ void gdn_token(Tile<K, V, NT>& t, Partials<V, NT>& red, int buf,
+                                          const float* q, const float* k, const float* v,
+                                          const QkScales& sc, float decay, float beta,
+                                          Before before, StoreO store_o) {
   using TL = Tile<K, V, NT>;
   const int tid = threadIdx.x;
   const int c4 = tid % TL::kLanesPerRow;  // column group (4 columns)
   const int r0 = tid / TL::kLanesPerRow;  // first row
   const int wid = tid / kWave;
-  __syncthreads();  // sm.q / sm.k / sm.v of this token are complete
-
   float pk[4] = {0.f, 0.f, 0.f, 0.f}, pq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < TL::kPasses; ++i) {
     const int r = r0 + i * TL::kRowsPerPass;
-    const float kr = sm.k[r], qr = sm.q[r];
+    const float kr = k[r], qr = q[r];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       t.h[i][c] *= decay;
@@ -158,40 +203,47 @@ __device__ __forceinline__ void gdn_token(Tile<K, V, NT>& t, Smem<K, V, NT>& sm,
     }
   }
   // Reduce over the rows held by the other lanes of this wave (same c4).
+  static_assert(TL::kLanesPerRow == 16 || TL::kLanesPerRow == 32, "rows of 64 or 128 columns");
 #pragma unroll
-  for (int o = TL::kLanesPerRow; o < kWave; o <<= 1)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      pk[c] += __shfl_xor(pk[c], o, kWave);
-      pq[c] += __shfl_xor(pq[c], o, kWave);
+  for (int c = 0; c < 4; ++c) {
+    if constexpr (TL::kLanesPerRow == 16) {
+      pk[c] = swap_sum<16>(pk[c]);
+      pq[c] = swap_sum<16>(pq[c]);
     }
+    pk[c] = swap_sum<32>(pk[c]);
+    pq[c] = swap_sum<32>(pq[c]);
+  }
+  typedef Vec<float, 4> V4;
   if ((tid % kWave) < TL::kLanesPerRow) {
+    *reinterpret_cast<V4*>(&red.p[buf][0][wid][c4 * 4]) = V4{{pk[0], pk[1], pk[2], pk[3]}};
+    *reinterpret_cast<V4*>(&red.p[buf][1][wid][c4 * 4]) = V4{{pq[0], pq[1], pq[2], pq[3]}};
+  }
+  before();
+  __syncthreads();
+  float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < NT / kWave; ++w) {
+    const V4 x = *reinterpret_cast<const V4*>(&red.p[buf][0][w][c4 * 4]);
+    const V4 y = *reinterpret_cast<const V4*>(&red.p[buf][1][w][c4 * 4]);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      sm.red[0][wid][c4 * 4 + c] = pk[c];
-      sm.red[1][wid][c4 * 4 + c] = pq[c];
+      a[c] += x.v[c];
+      b[c] += y.v[c];
     }
   }
-  __syncthreads();
-  if (tid < V) {
-    float a = 0.f, b = 0.f;
+  const V4 vv = *reinterpret_cast<const V4*>(&v[c4 * 4]);
+  float vn[4], o[4];
 #pragma unroll
-    for (int w = 0; w < NT / kWave; ++w) {
-      a += sm.red[0][w][tid];
-      b += sm.red[1][w][tid];
-    }
+  for (int c = 0; c < 4; ++c) {
     // v' = beta (v - h^T k);  o = h^T q + (k.q) v'
-    const float vn = beta * (sm.v[tid] - a);
-    sm.kh[tid] = vn;
-    store_o(tid, b + sm.scal[0] * vn);
+    const float n = beta * (vv.v[c] - sc.rk * a[c]);
+    o[c] = fmaf(sc.rq, b[c], sc.kq * n);
+    vn[c] = sc.rk * n;
   }
-  __syncthreads();
-  float vn[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) vn[c] = sm.kh[c4 * 4 + c];
+  if (r0 == 0) store_o(c4 * 4, o);
 #pragma unroll
   for (int i = 0; i < TL::kPasses; ++i) {
-    const float kr = sm.k[r0 + i * TL::kRowsPerPass];
+    const float kr = k[r0 + i * TL::kRowsPerPass];
 #pragma unroll
     for (int c = 0; c < 4; ++c) t.h[i][c] = fmaf(kr, vn[c], t.h[i][c]);
   }
@@ -237,47 +289,6 @@ __device__ __forceinline__ void store_tile(const Tile<K, V, NT>& t, float* base,
   }
 }
 
-// Loads q and k of one token (raw), then l2-normalises (optional) and
-// scales q.  Block-wide; ends with a barrier.
-template <int K, int V, int NT, typename LoadQK>
-__device__ __forceinline__ void prep_qk(Smem<K, V, NT>& sm, LoadQK load, bool l2norm,
-                                        float scale) {
-  const int tid = threadIdx.x;
-  // The previous token's readers of sm.q / sm.k / sm.scal are done.
-  __syncthreads();
-  if (tid < K) {
-    const float qv = load(0, tid), kv = load(1, tid);
-    sm.q[tid] = qv;
-    sm.k[tid] = kv;
-  }
-  __syncthreads();
-  if (tid < kWave) {
-    float sq = 0.f, sk = 0.f, kq = 0.f;
-    for (int i = tid; i < K; i += kWave) {
-      sq = fmaf(sm.q[i], sm.q[i], sq);
-      sk = fmaf(sm.k[i], sm.k[i], sk);
-      kq = fmaf(sm.q[i], sm.k[i], kq);
-    }
-    sq = group_sum<kWave>(sq);
-    sk = group_sum<kWave>(sk);
-    kq = group_sum<kWave>(kq);
-    if (tid == 0) {
-      const float rq = l2norm ? 1.0f / sqrtf(sq + 1e-6f) : 1.0f;
-      const float rk = l2norm ? 1.0f / sqrtf(sk + 1e-6f) : 1.0f;
-      sm.scal[1] = rq * scale;
-      sm.scal[2] = rk;
-      sm.scal[0] = kq * rq * rk * scale;  // (k_hat . q_hat) * scale
-    }
-  }
-  __syncthreads();
-  if (tid < K) {
-    sm.q[tid] *= sm.scal[1];
-    sm.k[tid] *= sm.scal[2];
-  }
-  // sm.q / sm.k are read by other lanes in gdn_token after its first
-  // barrier; sm.v must be written by the caller before that barrier too.
-}
-
 // ---------------------------------------------------------------------------
 // Recurrent GDN over varlen sequences.
 // ---------------------------------------------------------------------------
@@ -319,7 +330,13 @@ struct RecParams {
 template <int K, int V, typename T, typename GT, typename BT, int NS>
 __global__ void __launch_bounds__(kThreads) gdn_recurrent_kernel(RecParams p) {
   constexpr int VT = V / NS;
-  __shared__ Smem<K, VT> sm;
+  // Raw inputs of a token.  A wave reads token i's until it reaches the
+  // barrier of token i + 1, and those of token i + 1 are written before the
+  // barrier of token i: three buffers.
+  __shared__ __align__(16) struct {
+    float q[3][K], k[3][K], v[3][VT];
+  } in;
+  __shared__ __align__(16) Partials<VT> red;
   const int cs = static_cast<int>(blockIdx.x % NS);  // column slice
   const int64_t item = blockIdx.x / NS;
   const int64_t n = item / p.HV;
@@ -379,22 +396,37 @@ __global__ void __launch_bounds__(kThreads) gdn_recurrent_kernel(RecParams p) {
   // Per-token state writes: in place with a per-token slot column (2-D
   // indices or speculative decoding); otherwise once at the end.
   const bool per_token = p.inplace && p.idx && p.idx_s1 != 0;
+  auto put = [&](int buf, const TokIn& r) {
+    if (tid < K) {
+      in.q[buf][tid] = r.q;
+      in.k[buf][tid] = r.k;
+    }
+    if (tid < VT) in.v[buf][tid] = r.v;
+  };
+  put(0, cur);
+  __syncthreads();
+  int buf = 0;
   for (int64_t i = 0; i < len; ++i) {
     const int64_t tok = bos + i;
-    // The next token's inputs are fetched while this one computes.
+    const int next_buf = buf == 2 ? 0 : buf + 1;
+    // The next token's inputs are fetched while this one computes, and put in
+    // the next buffer ahead of this one's barrier.
     const TokIn nxt = i + 1 < len ? load_in(tok + 1) : cur;
-    prep_qk<K, VT>(sm, [&](int which, int) { return which == 0 ? cur.q : cur.k; },
-                   p.l2norm, p.scale);
-    if (tid < VT) sm.v[tid] = cur.v;
-    const float decay = __expf(cur.g);
-    const float beta = cur.b;
+    const QkScales sc = qk_scales<K>(in.q[buf], in.k[buf], p.l2norm, p.scale);
     T* o = reinterpret_cast<T*>(p.o) + (tok * p.HV + hv) * V + cs * VT;
-    gdn_token<K, VT>(t, sm, decay, beta, [&](int c, float val) { o[c] = from_f32<T>(val); });
+    gdn_token<K, VT>(
+        t, red, static_cast<int>(i & 1), in.q[buf], in.k[buf], in.v[buf], sc, __expf(cur.g), cur.b,
+        [&]() { put(next_buf, nxt); },
+        [&](int c, const float (&val)[4]) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) o[c + u] = from_f32<T>(val[u]);
+        });
     if (per_token) {
       const int64_t sl = slot_of(i);
       if (sl >= 0 && sl < p.slots) store_tile<K, VT>(t, p.ht + sl * p.ht_slot_stride + col0, V);
     }
     cur = nxt;
+    buf = next_buf;
   }
   if (!per_token) {
     if (p.inplace) {
@@ -553,9 +585,9 @@ __device__ __forceinline__ void conv8(const FusedParams& p, int64_t b, int64_t c
 template <int K, int V, typename T, typename GT, typename BT>
 __global__ void __launch_bounds__(kFusedThreads) gdn_conv_decode_kernel(FusedParams p) {
   constexpr int NT = kFusedThreads;
-  __shared__ Smem<K, V, NT> sm;
-  __shared__ float xv_lds[K * 2];          // q and k after conv + SiLU
-  __shared__ float vv_lds[16][V];          // v heads of the group (R <= 16)
+  __shared__ __align__(16) Partials<V, NT> red;
+  __shared__ __align__(16) float xv_lds[K * 2];  // q and k after conv + SiLU
+  __shared__ __align__(16) float vv_lds[16][V];          // v heads of the group (R <= 16)
   const int64_t b = blockIdx.x / p.H;
   const int h = static_cast<int>(blockIdx.x % p.H);
   const int R = p.HV / p.H;
@@ -628,6 +660,7 @@ __global__ void __launch_bounds__(kFusedThreads) gdn_conv_decode_kernel(FusedPar
   // while head j computes (two register tiles, unrolled by two): 204.4 ->
   // 197.8 us at config 5 on MI355X, the state stream no longer pausing
   // between the group's heads.
+  const QkScales sc = qk_scales<K>(xv_lds, xv_lds + K, p.l2norm, p.scale);
   Tile<K, V, NT> t2;
   auto head = [&](Tile<K, V, NT>& cur, Tile<K, V, NT>& nxt, int j) {
     const int hv = h * R + j;
@@ -635,18 +668,19 @@ __global__ void __launch_bounds__(kFusedThreads) gdn_conv_decode_kernel(FusedPar
     if (j + 1 < R) {
       if (st_ok) load_tile<K, V>(nxt, sbase + K * V); else zero_tile<K, V>(nxt);
     }
-    prep_qk<K, V>(sm, [&](int which, int e) { return xv_lds[which * K + e]; },
-                  p.l2norm, p.scale);
-    if (tid < V) sm.v[tid] = vv_lds[j][tid];
     float gv = ldf<GT>(p.g, b * p.HV + hv);
     float beta = p.beta ? ldf<BT>(p.beta, b * p.HV + hv) : 1.0f;
     if (p.gating) {
       gv = gdn_log_decay(gv + p.dt_bias[hv], p.A_log[hv], p.sp_beta, 1.0f / p.sp_beta, p.sp_thr);
       beta = sigmoid_exact(beta);
     }
-    const float decay = __expf(gv);
     T* o = reinterpret_cast<T*>(p.o) + (b * p.HV + hv) * V;
-    gdn_token<K, V>(cur, sm, decay, beta, [&](int c, float val) { o[c] = from_f32<T>(val); });
+    gdn_token<K, V>(
+        cur, red, j & 1, xv_lds, xv_lds + K, vv_lds[j], sc, __expf(gv), beta, [] {},
+        [&](int c, const float (&val)[4]) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) o[c + u] = from_f32<T>(val[u]);
+        });
     if (st_ok) store_tile<K, V>(cur, sbase);
   };
   for (int j = 0; j < R; j += 2) {
