@@ -717,7 +717,18 @@ int launch_varlen(VarlenParams p, xk_dtype dt, hipStream_t s) {
                       aligned(p.x, 2 * sizeof(T)) && aligned(p.out, 2 * sizeof(T));
     return pair ? launch_short_w<T, 2>(p, s) : launch_short_w<T, 1>(p, s);
   }
-  return vec ? launch_varlen_w<T, kV>(p, s) : launch_varlen_w<T, 1>(p, s);
+  if (!vec) return launch_varlen_w<T, 1>(p, s);
+  // 8 bytes of channels per lane, 4 where that makes at most two rounds of
+  // resident waves (8 on a SIMD).  A lane of 16 bytes holds weights, window
+  // and a run of tokens in 141 registers, 3 waves on a SIMD; 8 bytes take 82
+  // (5 waves) and 4 fewer still: small calls have too few waves to hide the
+  // chain of lookups, window and tokens, large ones then run their accesses
+  // too narrow.  MI355X, us per call at 16 / 8 / 4 bytes: 4,096 tokens x
+  // 2,048 bf16 channels 16.8 / 12.6 / 10.5, 8,192 x 4,096 37.4 / 31.6 / 26.5,
+  // 8,192 x 8,192 54.2 / 51.5 / 62.0, 16,384 x 8,192 95.9 / 95.8 / 123.
+  const int64_t waves = cdiv(p.D, kWave * (kV / 4)) * cdiv(p.num_tokens, kTileT);
+  if (waves <= int64_t{2} * 8 * 4 * num_cus()) return launch_varlen_w<T, kV / 4>(p, s);
+  return launch_varlen_w<T, kV / 2>(p, s);
 }
 
 }  // namespace
