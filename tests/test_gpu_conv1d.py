@@ -280,7 +280,7 @@ def test_v2_history_read_next_to_a_tile_edge(dev, W):
 
 # Batches of short sequences (one lane per sequence and channel pair): empty
 # and one-token sequences, lengths around the groups of four tokens and the
-# longest one sent there (32, and 33 past it); whole and partial 512-channel
+# longest ones sent there (8, or 24 with speculative windows); whole and partial 512-channel
 # blocks and odd channel counts; states contiguous, with channels apart, and
 # token-major; speculative windows and a padded slot.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -288,7 +288,8 @@ def test_v2_history_read_next_to_a_tile_edge(dev, W):
 @pytest.mark.parametrize("layout", ["dense", "apart", "token_major"])
 @pytest.mark.parametrize("lens,dim,W", [
     ([1] * 9, 1024, 4), ([4, 4, 4], 1030, 4), ([0, 1, 3, 5, 4, 8, 0], 513, 4),
-    ([32, 1, 31], 512, 4), ([33, 2], 512, 4), ([2, 3, 1], 520, 2), ([5, 6], 200, 6),
+    ([24, 1, 23], 512, 4), ([25, 2], 512, 4), ([8, 7], 512, 4), ([9, 2], 512, 4),
+    ([2, 3, 1], 520, 2), ([5, 6], 200, 6),
     ([3, 1], 7, 1)])
 def test_v2_short_sequences(dev, lens, dim, W, layout, spec, dtype):
     from torch_npu_ops_amd import ops

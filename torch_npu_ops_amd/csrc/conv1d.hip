@@ -520,21 +520,23 @@ __global__ void __launch_bounds__(256) conv1d_varlen_kernel(VarlenParams p) {
 // Varlen batches of short sequences (speculative verification, decode through
 // the varlen entry): one lane per (sequence, VEC channels), which loads the
 // window, the state entries it keeps and the first tokens at once, walks its
-// tokens and writes the state.  The tile kernel above has one lane per (16
-// tokens, 8 channels): a few sequences' tokens fill a fraction of the CUs
-// there, and each lane gathers and scatters the 2-byte state entries of all
-// its sequences one after the other.  Bound by the chain slot -> state ->
-// output at small batches; at 256 sequences of 8 drafts by its bytes (70% of
-// a copy's rate).  MI355X, 8192 bf16 channels, width 4, us per call, tile
+// tokens and writes the state.  The tile kernel has one lane per (16 tokens,
+// 2 to 4 channels): a few sequences' tokens fill a fraction of the CUs there,
+// and each lane gathers and scatters the 2-byte state entries of all its
+// sequences one after the other.  Bound by the chain slot -> state -> output
+// at small batches; at 256 sequences of 8 drafts by its bytes (70% of a
+// copy's rate).  MI355X, 8192 bf16 channels, width 4, us per call, tile
 // kernel -> this one (with direct state accesses in brackets):
-//   32 sequences of 1 token                142.3 -> 5.5 (5.7)
-//   32 of 4 tokens, speculative (6 entries) 75.0 -> 6.6 (8.2)
-//   256 of 8 tokens, speculative           213.2 -> 35.0 (79.5)
+//   32 sequences of 1 token                45.9 -> 5.5 (5.7)
+//   32 of 4 tokens, speculative (6 entries) 23.4 -> 6.6 (8.2)
+//   256 of 8 tokens, speculative            88.5 -> 34.2 (79.5)
 // ---------------------------------------------------------------------------
-// Longest sequence (as the caller declares it) sent here: a lane walks it
-// alone.  One sequence of 32 tokens takes 9.1 us here and 13.7 in the tile
-// kernel, one of 64 takes 13.8 and 13.9 and is left there.
-constexpr int64_t kShortLen = 32;
+// Longest sequence (as the caller declares it) sent here, where a lane walks
+// it alone.  32 sequences of 8 tokens take 7.1 us here and 11.5 in the tile
+// kernel, of 16 tokens 8.9 and 8.2; with speculative windows, whose states
+// grow with the draft, 32 of 16 take 11.5 and 28.7, 64 of 24 27.8 and 179,
+// 8 of 32 22.1 and 21.3.
+constexpr int64_t kShortLen = 8, kShortSpecLen = 24;
 constexpr int64_t kShortLds = 32768;  // most LDS for a block's states
 constexpr int kShortTok = 4;   // tokens loaded together
 constexpr int kShortKeep = 8;  // kept state entries loaded together
@@ -711,7 +713,8 @@ int launch_varlen(VarlenParams p, xk_dtype dt, hipStream_t s) {
   const bool vec = p.D % kV == 0 && p.sx % kV == 0 && p.so % kV == 0 &&
                    aligned(p.x, 16) && aligned(p.out, 16);
   p.w_vec = p.wdt == dt && p.swd == p.W && p.sww == 1 && aligned(p.w, 16);
-  if (p.max_query_len <= kShortLen && p.num_tokens <= kShortLen * p.B &&
+  const int64_t short_len = p.accepted ? kShortSpecLen : kShortLen;
+  if (p.max_query_len <= short_len && p.num_tokens <= short_len * p.B &&
       cdiv(p.D, 256) * p.B <= INT32_MAX) {
     const bool pair = p.D % 2 == 0 && p.sx % 2 == 0 && p.so % 2 == 0 &&
                       aligned(p.x, 2 * sizeof(T)) && aligned(p.out, 2 * sizeof(T));
