@@ -363,7 +363,9 @@ int xk_gdn_conv_gating_decode(
  *   256-byte aligned (chunk offsets + per-chunk inverse blocks).  For batches
  *   that leave most compute units idle behind long sequences the size
  *   includes room to run segments of them in parallel; a workspace that holds
- *   the rest but not that is accepted and runs every sequence in order.
+ *   the rest but not that is accepted and runs every sequence in order, and
+ *   so does a call with final_state == initial_state (the state updated in
+ *   place; the two must be the same or not overlap).
  */
 int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                      int64_t HV);

@@ -125,3 +125,50 @@ def test_nan_value_spreads_no_further(dev):
     a, b = _run(dev, q, k, v, g, beta, h0, cu), _run(dev, q, k, v, g, beta, h0, cu, segments=False)
     assert b[1][:, 1, :, 17].isnan().all() and not b[1][:, 1, :, 64:].isnan().any()
     _same(a, b)
+
+
+def _least_workspace(T, N, HV):
+    """Bytes of workspace that a call cannot do without: the chunk and
+    sequence tables, the 8 KiB store sink and a record of 19,712 bytes per
+    (chunk, v-head).  What a segmented call uses beyond them starts there."""
+    def align(n):
+        return (n + 255) // 256 * 256
+    nt = T // 64 + N
+    return align(4 * (N + 1)) + align(4 * N) + align(8 * nt) + 8192 + nt * HV * 19712
+
+
+def _call(t, fin, h0, ws, ws_bytes, V=128, l2norm=True):
+    """One xk_gdn_chunk_fwd on device tensors t = (q, k, v, g, beta, cu)."""
+    from torch_npu_ops_amd import _lib, ops
+    q, k, v, g, beta, cu = t
+    T, H, HV, N = q.shape[1], q.shape[2], v.shape[2], cu.numel() - 1
+    o = torch.empty_like(v)
+    st = _lib.lib().xk_gdn_chunk_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.XK_BF16, g.data_ptr(), _lib.XK_F32,
+        beta.data_ptr(), _lib.XK_BF16, o.data_ptr(), h0.data_ptr(), fin.data_ptr(), cu.data_ptr(),
+        _lib.XK_I32, N, T, H, HV, 128, V, 128 ** -0.5, int(l2norm), ws.data_ptr(), ws_bytes,
+        ops._stream(o))
+    _lib.check(st, "xk_gdn_chunk_fwd")
+    return o
+
+
+@pytest.mark.parametrize("lens,H,HV", [([2111], 1, 2), ([64 * 31 + 1, 0, 1, 700], 2, 4)])
+def test_state_in_place_runs_in_order(dev, lens, H, HV):
+    """final_state == initial_state: the first segment of a sequence reads the
+    buffer that its last one writes, so the call must not be segmented (the
+    workspace past the least is left alone) and is bit for bit the in-order
+    call on separate buffers."""
+    from torch_npu_ops_amd import _lib
+    q, k, v, g, beta, h0, cu = _inputs(lens, H, HV, seed=11)
+    t = [x.to(dev).contiguous() for x in (q, k, v, g, beta, cu)]
+    T, N = sum(lens), len(lens)
+    need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV), _least_workspace(T, N, HV)
+    assert need > least
+    start = h0.to(dev)
+    fin = torch.empty_like(start)
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
+    want = _call(t, fin, start, ws, least)
+    state = start.clone()
+    got = _call(t, state, state, ws, need)
+    assert torch.equal(got, want) and torch.equal(state, fin)
+    assert (ws[least:] == 0xA5).all()

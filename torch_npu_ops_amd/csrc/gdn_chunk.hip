@@ -1573,7 +1573,15 @@ extern "C" int xk_gdn_chunk_fwd_strided(
   p.HV = static_cast<int>(HV);
   p.scale = scale;
   p.l2norm = use_qk_l2norm;
-  const SegPlan plan = seg_plan(total_tokens, N, HV, K, V);
+  // Segments of a sequence run side by side, the first from the initial state
+  // while the last writes the final state: where the two overlap (a state
+  // updated in place), whole sequences run, whose blocks each read their part
+  // of the state before they write it.
+  const uintptr_t s0 = reinterpret_cast<uintptr_t>(initial_state),
+                  s1 = reinterpret_cast<uintptr_t>(final_state);
+  const uintptr_t state_bytes = static_cast<uintptr_t>(N * HV * K * V) * 4;
+  const bool in_place = s0 && s1 && s0 < s1 + state_bytes && s1 < s0 + state_bytes;
+  const SegPlan plan = in_place ? SegPlan{} : seg_plan(total_tokens, N, HV, K, V);
   if (plan.segs && static_cast<int64_t>(workspace_bytes) >= need + plan.bytes) {
     char* seg = p.rec + p.NTmax * HV * kRec;
     p.seg_max = plan.segs;
