@@ -109,10 +109,11 @@ struct ChunkParams {
   int seg_max;        // segments the workspace holds
   int seg_cus, seg_nvt;  // compute units and V tiles the plan counts on
   int32_t* seg_len;   // the plan: chunks per segment
-  char* seg_m;        // [seg_max, HV]: transition of a segment, kSegImg bytes of operand images
+  char* seg_m;        // [seg_max, HV]: transition M - c I of a segment, kSegImg bytes of operand images
+  float* seg_c;       // [seg_max, HV]: c, the product of the segment's decays
   float* seg_b;       // [seg_max, HV, K, V]: its end state from zero (the first one's: from h0),
                       // then the state after it
-  int32_t* seg_over;  // [seg_max, HV, 2]: a transition entry of that half exceeds kSegLimit
+  int32_t* seg_over;  // [seg_max, HV, 2]: an entry of that half of M - c I, or c, exceeds kSegLimit
   int32_t* seg_bad;   // [N, HV]: the head runs in order
 };
 
@@ -129,7 +130,8 @@ __device__ __forceinline__ char* rec_at(const ChunkParams& p, int64_t c, int hv)
 //    M (the same recurrence without values, from the identity: K more
 //    columns), without outputs;
 //  * gdn_chunk_combine_kernel: the states at the segment boundaries,
-//    S <- M_i S + B_i in order;
+//    S <- M_i S + B_i in order, as c_i S + (M_i - c_i I) S + B_i with c_i the
+//    product of the segment's decays, to fp32 precision;
 //  * kSegOut: every segment from its entry state, with outputs.
 // The work of the state pass grows about 2.4 times, so this pays only where
 // the chip is idle.  len is chosen on the device, where the lengths are
@@ -141,20 +143,27 @@ __device__ __forceinline__ char* rec_at(const ChunkParams& p, int64_t c, int hv)
 // tokens in all, 16 v-heads: 173 -> 142.  A batch that is offered the passes
 // but keeps whole sequences pays about 4 us for the two idle launches.
 //
-// A transition entry outside [-kSegLimit, kSegLimit] (or NaN) makes the whole
-// head run in order: with keys of norm <= 1, beta in [0, 1] and decays <= 1 a
-// transition has norm <= 1 and its products lose nothing; without these they
-// could overflow or cancel where the chain in order does not.
+// A chunk of the chain in order scales the state in fp32 and rounds only what
+// the delta rule adds (bf16 hi/lo operands).  A boundary must lose no more:
+// M in hi/lo images would round the whole state to 2^-17 there however little
+// the segment changes it (final states of heads with beta ~ 0.01 and decays
+// ~ 1e-5 a token were 15 to 30 times as far from 64 bits as in order).  With
+// c split off and 24-bit products the errors of the two are the same.
+//
+// An entry of M - c I (or c) outside [-kSegLimit, kSegLimit] (or NaN) makes
+// the whole head run in order: with keys of norm <= 1, beta in [0, 1] and
+// decays <= 1 a transition has norm <= 1; without these its products could
+// overflow or cancel where the chain in order does not.
 // ---------------------------------------------------------------------------
 constexpr float kSegLimit = 2.f;
-constexpr int64_t kSegImg = 128 * 128 * 4;  // bf16 hi and lo images of one transition
+constexpr int64_t kSegImg = 128 * 128 * 6;  // three bf16 images of one transition's operands
 constexpr int64_t kSegSeqs = 16;            // most sequences (the plan loops over them)
 
 // Time of the state pass (us) when the longest sequence is cut into `s`
 // segments of `len` chunks: `sums` kSegSum blocks and `outs` kSegOut blocks,
 // each on one CU at a time.  A step takes 1.6 (sum) or 2.35 us (out) on an
 // idle chip and about 0.6 us more on a full one, a step of the combine
-// kernel 1.2 us (measured on MI355X; the model is within 5% of the measured
+// kernel 1.4 us (measured on MI355X; the model is within 5% of the measured
 // passes from 2,048 to 32,768 tokens).  `exact`: the block counts are known,
 // so that a round of blocks that is nearly empty counts as one.
 __host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, int cus,
@@ -164,7 +173,7 @@ __host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, in
     return fmaxf(1.f, exact ? ceilf(load) : load) * len * (step + 0.6f * fminf(1.f, load));
   };
   const float out = 8.f + time(outs, 2.35f);
-  return s <= 1 ? out : out + 14.f + time(sums, 1.6f) + 1.2f * (s - 2);
+  return s <= 1 ? out : out + 14.f + time(sums, 1.6f) + 1.4f * (s - 2);
 }
 
 // Chunks per segment for this batch, 0 for whole sequences (wave-uniform; N <=
@@ -1075,6 +1084,7 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     store_fac(sm.fac[0], opsA.fac);
   }
   __syncthreads();
+  float decay = 1.f;  // kSegSum: product of the chunks' e^{g_last}, rounded as the state's is
 
   auto step = [&](const EarlyOps8& cur, EarlyOps8& nxt, int64_t ci) {
     const int64_t s = bos + ci * kC;
@@ -1188,6 +1198,7 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
       }
     }
     if constexpr (kOut) load_out8(outo, cidx0 + cn);
+    if constexpr (!kOut) decay *= cur.egl;
 
     __builtin_amdgcn_iglp_opt(0);
 #pragma unroll
@@ -1222,24 +1233,40 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
     if (ci + 1 < nch) step(opsB, opsA, ci + 1);
   }
   if (is_m) {
-    // Transition columns scol .. + 63 as A operands of the combine kernel
-    // (image (w, kk), hi then lo: rows 16 w + l % 16, columns 32 kk + 8 (l /
-    // 16) .. + 7), read transposed from the state's bf16 copy.
-    bool over = false;
-    char* img = p.seg_m + sh * kSegImg + (wid * KK + scol / 32) * 2048 + 16 * lane;
+    // M - c I, columns scol .. + 63, as A operands of the combine kernel, each
+    // value in three bf16 parts: image (w, q, part) holds rows 16 w + l % 16
+    // and, in the 16 bytes of lane l, columns 32 q + 4 (l / 16) + {0 .. 3, 16
+    // .. 19}.  Quads transpose their 4 x 4 blocks of the MFMA layout for it.
+    bool over = !(fabsf(decay) <= kSegLimit);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int m2 = 0; m2 < M2; ++m2) {
+      bf8_t part[3];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r0 = 32 * kk + 8 * lg;
-        const bf8_t x = cat_bf8(sb8_col4(sm.sb[h], 16 * wid, r0), sb8_col4(sm.sb[h], 16 * wid, r0 + 4));
-        *reinterpret_cast<bf8_t*>(img + 2048 * kk + 1024 * h) = x;
-        if (h == 0)
+      for (int nj = 0; nj < NJ; ++nj) {
+        f4_t x = sreg[m2][nj];
+        const int kr = wr * (K / 4) + m2 * 16 + 4 * lg, col = scol + cb + nj * 16 + l15;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) over |= !(fabsf(static_cast<float>(x[e])) <= kSegLimit);
+        for (int i = 0; i < 4; ++i) {
+          if (kr + i == col) x[i] -= decay;
+          over |= !(fabsf(x[i]) <= kSegLimit);
+        }
+        Vec<__bf16, 4> t[3];
+        split4x3(quad_transpose(x), t);
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) part[u][4 * nj + i] = t[u].v[i];
       }
+      char* img = p.seg_m + sh * kSegImg + ((wr * M2 + m2) * KK + (scol + cb) / 32) * 3072 +
+                  16 * (16 * (l15 >> 2) + 4 * lg + (lane & 3));
+#pragma unroll
+      for (int u = 0; u < 3; ++u) *reinterpret_cast<bf8_t*>(img + 1024 * u) = part[u];
+    }
     const int any = __syncthreads_or(over);
-    if (tid == 0) p.seg_over[2 * sh + (vt - nvt)] = any;
+    if (tid == 0) {
+      p.seg_over[2 * sh + (vt - nvt)] = any;
+      if (vt == nvt) p.seg_c[sh] = decay;
+    }
   } else if (s_out) {
 #pragma unroll
     for (int m2 = 0; m2 < M2; ++m2)
@@ -1256,18 +1283,21 @@ gdn_chunk_state8_kernel(ChunkParams p, int nvt) {
 
 // ---------------------------------------------------------------------------
 // States at the segment boundaries of one (sequence, v-head, 16 V columns):
-// S_1 = the state after segment 0, S_{i+1} = M_i S_i + B_i; S_{i+1} replaces
-// B_i.  A block of eight waves; wave w owns state rows 16 w .. + 15.  A step
-// is bound by its 64 KB of operand images into one CU and takes 1.2 us
-// (2.2 us with M in fp32, split here by every column tile; as a prologue of
-// the kSegOut blocks, whose 64 columns need each image in two waves, 2.5 us).
+// S_1 = the state after segment 0, S_{i+1} = c_i S_i + (M_i - c_i I) S_i +
+// B_i; S_{i+1} replaces B_i.  A block of eight waves; wave w owns state rows
+// 16 w .. + 15.  Both factors of the product enter in three bf16 parts, so it
+// is good to 2^-24 (see "Segments").  A step waits for its 96 KB of operand
+// images, read 2 to 3 us ahead into registers: 1.4 us (two parts: 64 KB and
+// 1.0 us, but 2^-17; fp32 images and MFMA: 64 KB, 2.0 us of matrix time).
+// Two steps in flight instead of three take 1.7 us a step.
 // ---------------------------------------------------------------------------
 template <int K>
 __global__ void __launch_bounds__(kTh8) gdn_chunk_combine_kernel(ChunkParams p, int V) {
   static_assert(K == 128, "eight waves of 16 rows");
   constexpr int KK = K / 32;
   constexpr int kDepth = 3;  // steps whose operands are in flight
-  __shared__ __align__(16) __bf16 sb[2][2][16 * K];  // state hi / lo [v][k], double-buffered
+  // The state's three parts [v][k], double-buffered; keys in the images' order.
+  __shared__ __align__(16) __bf16 sb[2][3][16 * K];
   const int lane = threadIdx.x & 63, wid = wave_index();
   const int l15 = lane & 15, lg = lane >> 4;
   const int nt = V / 16;
@@ -1292,29 +1322,32 @@ __global__ void __launch_bounds__(kTh8) gdn_chunk_combine_kernel(ChunkParams p, 
     if (lane == 0) p.seg_bad[item] = any != 0;
   }
   const int r4 = 16 * wid + 4 * lg;  // first of the lane's four state rows
+  const int kpos = 32 * (wid >> 1) + 8 * lg + 4 * (wid & 1);  // their place in the images' order
   // Per-step strides and the lane's place in each, so that a step's
   // addresses are one scalar base plus one lane offset.
   float* bseg = p.seg_b + sh0 * K * V;
   const int64_t bstep = static_cast<int64_t>(p.HV) * K * V;
   const uint32_t boff = static_cast<uint32_t>(r4) * V + v0 + l15;
-  const char* mseg = p.seg_m + sh0 * kSegImg + wid * (2 * KK * 1024);
+  const char* mseg = p.seg_m + sh0 * kSegImg + wid * (KK * 3072);
   const int64_t mstep = static_cast<int64_t>(p.HV) * kSegImg;
   struct Stage {
-    bf8_t mh[KK], ml[KK];
+    bf8_t m[KK][3];
     f4_t b;
+    float c;
   } st[kDepth];
   auto load_b = [&](int i) {
     const float* b = bseg + i * bstep;
     return f4_t{b[boff], b[boff + V], b[boff + 2 * V], b[boff + 3 * V]};
   };
   auto load = [&](Stage& t, int i) {
+    t.c = p.seg_c[sh0 + static_cast<int64_t>(i) * p.HV];
     t.b = load_b(i);
     const char* m = mseg + i * mstep;
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      t.mh[kk] = *reinterpret_cast<const bf8_t*>(m + 2048 * kk + 16u * lane);
-      t.ml[kk] = *reinterpret_cast<const bf8_t*>(m + 2048 * kk + 1024 + 16u * lane);
-    }
+    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        t.m[kk][u] = *reinterpret_cast<const bf8_t*>(m + 3072 * kk + 1024 * u + 16u * lane);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto store = [&](int i, const f4_t& v) {
@@ -1336,26 +1369,31 @@ __global__ void __launch_bounds__(kTh8) gdn_chunk_combine_kernel(ChunkParams p, 
   }
   auto step = [&](Stage& t, int i) {
     const int buf = i & 1;
-    Vec<__bf16, 4> h, l;
-    split4(s, h, l);
-    *reinterpret_cast<Vec<__bf16, 4>*>(&sb[buf][0][sb8_off(l15, r4)]) = h;
-    *reinterpret_cast<Vec<__bf16, 4>*>(&sb[buf][1][sb8_off(l15, r4)]) = l;
+    Vec<__bf16, 4> part[3];
+    split4x3(s, part);
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      *reinterpret_cast<Vec<__bf16, 4>*>(&sb[buf][u][sb8_off(l15, kpos)]) = part[u];
     store(i - 1, s);
     // State copy complete; the other buffer's readers passed the barrier before.
     __syncthreads();
-    f4_t c = {0.f, 0.f, 0.f, 0.f};
-    s = t.b;
+    // Parts h, m, l of each: every product but m l, l m and l l (2^-24).
+    f4_t acc[3] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
-      const bf8_t sh = *reinterpret_cast<const bf8_t*>(&sb[buf][0][sb8_off(l15, 32 * kk + 8 * lg)]);
-      const bf8_t sl = *reinterpret_cast<const bf8_t*>(&sb[buf][1][sb8_off(l15, 32 * kk + 8 * lg)]);
-      s = mfma16(t.mh[kk], sh, s);
-      c = mfma16(t.mh[kk], sl, c);
-      c = mfma16(t.ml[kk], sh, c);
+      bf8_t x[3];
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        x[u] = *reinterpret_cast<const bf8_t*>(&sb[buf][u][sb8_off(l15, 32 * kk + 8 * lg)]);
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+#pragma unroll
+        for (int w = 0; w + u < 3; ++w) acc[u + w] = mfma16(t.m[kk][w], x[u], acc[u + w]);
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = fmaf(t.c, s[e], t.b[e]) + (acc[0][e] + (acc[1][e] + acc[2][e]));
     __builtin_amdgcn_sched_barrier(0);
     load(t, min(i + kDepth, last));
-    s += c;
   };
   int i = 1;
   for (; i + kDepth - 1 <= last; i += kDepth) {
@@ -1456,7 +1494,7 @@ SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t
   // Several sequences: room for one round of kSegOut blocks.
   if (r.segs && N > 1) r.segs = static_cast<int>(std::max<int64_t>(r.segs, cus / tiles) + N / 2);
   if (r.segs)
-    r.bytes = 256 + align256(4 * N * HV) + align256(8 * r.segs * HV) +
+    r.bytes = 256 + align256(4 * N * HV) + align256(8 * r.segs * HV) + align256(4 * r.segs * HV) +
               r.segs * HV * (kSegImg + K * V * 4);
   return r;
 }
@@ -1593,6 +1631,8 @@ extern "C" int xk_gdn_chunk_fwd_strided(
     seg += align256(4 * N * HV);
     p.seg_over = reinterpret_cast<int32_t*>(seg);
     seg += align256(8 * plan.segs * HV);
+    p.seg_c = reinterpret_cast<float*>(seg);
+    seg += align256(4 * plan.segs * HV);
     p.seg_m = seg;
     p.seg_b = reinterpret_cast<float*>(seg + plan.segs * HV * kSegImg);
   }

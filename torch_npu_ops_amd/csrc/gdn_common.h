@@ -60,6 +60,18 @@ __device__ __forceinline__ void split4(const f4_t& x, Vec<__bf16, 4>& h, Vec<__b
   l.v[3] = l1[1];
 }
 
+// Four values in three bf16 parts (24 mantissa bits).
+__device__ __forceinline__ void split4x3(const f4_t& x, Vec<__bf16, 4> (&p)[3]) {
+  f4_t r = x;
+#pragma unroll
+  for (int u = 0; u < 3; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[u].v[i] = static_cast<__bf16>(r[i]);
+      r[i] -= static_cast<float>(p[u].v[i]);
+    }
+}
+
 // Eight values split into hi / lo.
 __device__ __forceinline__ void split8(const f4_t& a, const f4_t& b, bf8_t& h, bf8_t& l) {
 #pragma unroll
@@ -252,6 +264,24 @@ __device__ __forceinline__ bf8_t kr_a(const __bf16* kr, int wid, int kk) {
 
 // Column 16 mi + lane % 16 of the tile at rows r0 .. r0 + 3 (r0 may differ
 // between the 16-lane groups, not within one), as 4 bf16 bit patterns.
+// Transpose of the 4 x 4 blocks (register i, lane b of a quad) -> (register
+// b, lane i), in two exchanges as q4_to_a's.
+template <int CTRL>
+__device__ __forceinline__ float quad_dpp_f32(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ f4_t quad_transpose(const f4_t& r) {
+  const bool b0 = threadIdx.x & 1, b1 = (threadIdx.x >> 1) & 1;
+  constexpr int kXor1 = 0xB1, kXor2 = 0x4E;  // quad_perm(1,0,3,2), (2,3,0,1)
+  const float x0 = quad_dpp_f32<kXor2>(r[0]), x1 = quad_dpp_f32<kXor2>(r[1]);
+  const float x2 = quad_dpp_f32<kXor2>(r[2]), x3 = quad_dpp_f32<kXor2>(r[3]);
+  const float s0 = b1 ? x2 : r[0], s2 = b1 ? r[2] : x0;
+  const float s1 = b1 ? x3 : r[1], s3 = b1 ? r[3] : x1;
+  const float y0 = quad_dpp_f32<kXor1>(s0), y1 = quad_dpp_f32<kXor1>(s1);
+  const float y2 = quad_dpp_f32<kXor1>(s2), y3 = quad_dpp_f32<kXor1>(s3);
+  return f4_t{b0 ? y1 : s0, b0 ? s1 : y0, b0 ? y3 : s2, b0 ? s3 : y2};
+}
 typedef short s4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ s4_t kr_col4(const __bf16* kr, int mi, int r0) {
   typedef __attribute__((address_space(3))) s4_t lds_s4;
