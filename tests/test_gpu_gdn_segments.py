@@ -152,7 +152,7 @@ def _call(t, fin, h0, ws, ws_bytes, V=128, l2norm=True):
     return o
 
 
-@pytest.mark.parametrize("lens,H,HV", [([2111], 1, 2), ([64 * 31 + 1, 0, 1, 700], 2, 4)])
+@pytest.mark.parametrize("lens,H,HV", [([2111], 1, 2), ([64 * 63 + 1, 0, 1, 1900], 2, 4)])
 def test_state_in_place_runs_in_order(dev, lens, H, HV):
     """final_state == initial_state: the first segment of a sequence reads the
     buffer that its last one writes, so the call must not be segmented (the
@@ -163,7 +163,7 @@ def test_state_in_place_runs_in_order(dev, lens, H, HV):
     t = [x.to(dev).contiguous() for x in (q, k, v, g, beta, cu)]
     T, N = sum(lens), len(lens)
     need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV), _least_workspace(T, N, HV)
-    assert need > least
+    assert need > least + 256  # room for segments
     start = h0.to(dev)
     fin = torch.empty_like(start)
     ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
@@ -220,3 +220,33 @@ def test_slow_heads_lose_no_precision(dev, beta_to, decay_to, mean):
         err[name] = ((fin.cpu().double() - exact).norm() / exact.norm()).item()
     print(err)
     assert err["segments"] <= 2 * err["order"]
+
+
+# A batch that is offered the segment passes takes them whatever its lengths
+# (idle passes would slow it down), from the shortest chains that are offered
+# them to many segments; a batch whose equal lengths would gain nothing is not.
+@pytest.mark.parametrize("N,HV,T,offered", [
+    (1, 8, 1024, True), (1, 24, 2048, True), (2, 16, 4096, True), (4, 8, 8192, True),
+    (6, 4, 12288, True), (16, 1, 16384, True), (1, 24, 1024, False), (2, 16, 2048, False),
+    (2, 24, 4096, False), (4, 16, 8192, False), (6, 8, 6144, False)])
+@pytest.mark.parametrize("kind", ["equal", "ragged", "one_long"])
+def test_offered_segments_are_taken(dev, N, HV, T, offered, kind):
+    from torch_npu_ops_amd import _lib
+    need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV), _least_workspace(T, N, HV)
+    assert (need > least + 256) == offered
+    if not offered:
+        return
+    if kind == "equal":
+        lens = [T // N] * N
+    elif kind == "ragged":
+        lens = [max(1, 2 * T * (i + 1) // (N * (N + 1))) for i in range(N)]
+    else:
+        lens = [1] * N
+    lens[-1] += T - sum(lens)
+    q, k, v, g, beta, h0, cu = _inputs(lens, 1, HV, seed=T)
+    t = [x.to(dev).contiguous() for x in (q, k, v, g, beta, cu)]
+    h0 = h0.to(dev)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    _call(t, torch.empty_like(h0), h0, ws, need)
+    per = int(ws[least:least + 4].view(torch.int32))  # chunks per segment
+    assert 0 < per < (max(lens) + 63) // 64

@@ -137,11 +137,10 @@ __device__ __forceinline__ char* rec_at(const ChunkParams& p, int64_t c, int hv)
 // the chip is idle.  len is chosen on the device, where the lengths are
 // known: one block of the prep kernel evaluates seg_cost for 1 .. 64
 // segments of the longest sequence, one candidate per lane.  The host
-// launches these passes if a batch of this size can gain (seg_plan).
-// MI355X, us per call of the whole op, one sequence of 8 v-heads: 4,096 tokens
-// 174.9 -> 74.1, 32,768 tokens 1266 -> 276; 4 ragged sequences of 8,192
-// tokens in all, 16 v-heads: 173 -> 142.  A batch that is offered the passes
-// but keeps whole sequences pays about 4 us for the two idle launches.
+// launches these passes if a batch of this size gains whatever its lengths
+// (seg_plan).  MI355X, us per call of the whole op without and with segments:
+// one sequence of 8 v-heads, 1,024 tokens 52 and 50, 4,096 tokens 175 and 77,
+// 32,768 tokens 1266 and 280; 2 sequences of 4,096 x 16 v-heads 180 and 140.
 //
 // A chunk of the chain in order scales the state in fp32 and rounds only what
 // the delta rule adds (bf16 hi/lo operands).  A boundary must lose no more:
@@ -160,17 +159,18 @@ constexpr int64_t kSegImg = 128 * 128 * 6;  // three bf16 images of one transiti
 constexpr int64_t kSegSeqs = 16;            // most sequences (the plan loops over them)
 
 // Time of the state pass (us) when the longest sequence is cut into `s`
-// segments of `len` chunks: `sums` kSegSum blocks and `outs` kSegOut blocks,
-// each on one CU at a time.  A step takes 1.6 (sum) or 2.35 us (out) on an
-// idle chip and about 0.6 us more on a full one, a step of the combine
-// kernel 1.4 us (measured on MI355X; the model is within 5% of the measured
-// passes from 2,048 to 32,768 tokens).  `exact`: the block counts are known,
-// so that a round of blocks that is nearly empty counts as one.
-__host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, int cus,
-                                          bool exact) {
+// segments of `len` chunks: `sums` kSegSum blocks and `outs` kSegOut blocks in
+// rounds of one per CU.  `sums` includes the transition blocks of first
+// segments, which end at once: an XCD hands its blocks to its shader engines
+// in turn, and with four tiles per (segment, head) all of one kind fall to
+// one engine, so the places that idle blocks leave are not taken by others
+// (3 segments x 24 heads, 240 blocks of 288 with work, take two rounds of 256
+// CUs).  A step takes 1.6 (sum) or 2.35 us (out) on an idle chip and about
+// 0.6 us more on a full one, a step of the combine kernel 1.4 us.
+__host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, int cus) {
   auto time = [&](int blocks, float step) {
     const float load = static_cast<float>(blocks) / cus;
-    return fmaxf(1.f, exact ? ceilf(load) : load) * len * (step + 0.6f * fminf(1.f, load));
+    return fmaxf(1.f, ceilf(load)) * len * (step + 0.6f * fminf(1.f, load));
   };
   const float out = 8.f + time(outs, 2.35f);
   return s <= 1 ? out : out + 14.f + time(sums, 1.6f) + 1.4f * (s - 2);
@@ -185,14 +185,11 @@ __device__ __forceinline__ int wave_seg_len(const ChunkParams& p) {
   int longest = 1;
   for (int n = 0; n < N; ++n) longest = max(longest, __builtin_amdgcn_readlane(w.cnt, n));
   const int len = (longest + lane) / (lane + 1);
-  int segs = 0, ms = 0;
-  for (int n = 0; n < N; ++n) {
-    const int c = (__builtin_amdgcn_readlane(w.cnt, n) + len - 1) / len;
-    segs += max(c, 1);
-    ms += max(c - 2, 0);
-  }
-  const float cost = seg_cost(lane + 1, len, ((segs - N) * p.seg_nvt + ms * 2) * p.HV,
-                              segs * p.seg_nvt * p.HV, p.seg_cus, true);
+  int segs = 0;
+  for (int n = 0; n < N; ++n)
+    segs += max((__builtin_amdgcn_readlane(w.cnt, n) + len - 1) / len, 1);
+  const float cost = seg_cost(lane + 1, len, (segs - N) * (p.seg_nvt + 2) * p.HV,
+                              segs * p.seg_nvt * p.HV, p.seg_cus);
   // Smallest cost, the fewest segments among equals.
   int key = lane == 0 || segs <= p.seg_max ? static_cast<int>(fminf(cost * 16.f, 3e7f)) : 30000000;
   key = key * kWave + lane;
@@ -1460,32 +1457,31 @@ int chunk_beta(const ChunkParams& p, int64_t V, xk_dtype bdt, hipStream_t s) {
 int64_t nt_max(int64_t total_tokens, int64_t N) { return total_tokens / kC + N; }
 
 // Whether a call takes the segmented state pass, and its workspace past the
-// records.  The lengths are not known here: several sequences are taken to
-// be ragged (the longest 1.5 times their mean), one is known exactly.
+// records.  The lengths are not known here.  Several sequences are taken to
+// be equally long, where segments gain least: with the same tokens a longer
+// sequence lengthens the chain in order and leaves the segments' work as it
+// is, so a batch that is offered the passes always takes them.  (Two idle
+// passes cost 3 to 4 us, 3% of 4 equal sequences of 2,048 tokens x 16
+// v-heads, more than it is right to take from batches that cannot gain.)
+constexpr int64_t kSegHead = 256;  // the plan's word; always part of the size
 struct SegPlan {
   int segs = 0;  // most segments; 0: whole sequences
-  int64_t bytes = 0;
+  int64_t bytes = kSegHead;
 };
 SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t V) {
   SegPlan r;
   const int cus = num_cus();
   const int64_t tiles = HV * (V / 64);
-  // Several sequences that fill over half the chip leave no whole round of
-  // blocks to gain (3 sequences of 32 v-heads: 409 us without, 433 with).
-  if (N <= 0 || N > kSegSeqs || V % 64 != 0 || N * tiles * (N > 1 ? 2 : 1) > cus) return r;
-  const int64_t chunks = cdiv(total_tokens, kC);
-  const int64_t longest = N == 1 ? chunks : cdiv(3 * chunks, 2 * N);
+  if (N <= 0 || N > kSegSeqs || V % 64 != 0 || N * tiles > cus) return r;
+  const int64_t longest = std::max<int64_t>(cdiv(cdiv(total_tokens, N), kC), 1);
   auto cost = [&](int s, int64_t len, int64_t sums, int64_t outs) {
-    return seg_cost(s, static_cast<int>(len), static_cast<int>(std::max<int64_t>(sums, 0)),
-                    static_cast<int>(outs), cus, N == 1);
+    return seg_cost(s, static_cast<int>(len), static_cast<int>(sums), static_cast<int>(outs), cus);
   };
-  float best = cost(1, longest, 0, N * tiles);
-  if (N > 1) best -= 4.f;  // what the passes cost a batch that turns out not to gain
+  // (At least 2 us must be gained: the model is good to a few percent.)
+  float best = cost(1, longest, 0, N * tiles) - 2.f;
   for (int s = 2; s <= 64; ++s) {
-    const int64_t len = cdiv(longest, s);
-    const int64_t segs = N == 1 ? cdiv(chunks, len) : chunks / len + N / 2;
-    const int64_t sums = (segs - N) * (tiles + 2 * HV) - (N == 1 ? 2 : N) * HV;
-    const float c = cost(s, len, sums, segs * tiles);
+    const int64_t len = cdiv(longest, s), segs = N * cdiv(longest, len);
+    const float c = cost(s, len, (segs - N) * (tiles + 2 * HV), segs * tiles);
     if (c < best) {
       best = c;
       r.segs = static_cast<int>(segs);
@@ -1494,7 +1490,7 @@ SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t
   // Several sequences: room for one round of kSegOut blocks.
   if (r.segs && N > 1) r.segs = static_cast<int>(std::max<int64_t>(r.segs, cus / tiles) + N / 2);
   if (r.segs)
-    r.bytes = 256 + align256(4 * N * HV) + align256(8 * r.segs * HV) + align256(4 * r.segs * HV) +
+    r.bytes = kSegHead + align256(4 * N * HV) + align256(8 * r.segs * HV) + align256(4 * r.segs * HV) +
               r.segs * HV * (kSegImg + K * V * 4);
   return r;
 }
@@ -1626,7 +1622,7 @@ extern "C" int xk_gdn_chunk_fwd_strided(
     p.seg_cus = num_cus();
     p.seg_nvt = static_cast<int>(V / 64);
     p.seg_len = reinterpret_cast<int32_t*>(seg);
-    seg += 256;
+    seg += kSegHead;
     p.seg_bad = reinterpret_cast<int32_t*>(seg);
     seg += align256(4 * N * HV);
     p.seg_over = reinterpret_cast<int32_t*>(seg);
