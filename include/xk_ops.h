@@ -362,10 +362,10 @@ int xk_gdn_conv_gating_decode(
  *   workspace >= xk_gdn_chunk_workspace_bytes(total_tokens, N, HV) bytes,
  *   256-byte aligned (chunk offsets + per-chunk inverse blocks).  For batches
  *   that leave most compute units idle behind long sequences the size
- *   includes room to run segments of them in parallel; a workspace that holds
- *   the rest but not that is accepted and runs every sequence in order, and
- *   so does a call with final_state == initial_state (the state updated in
- *   place; the two must be the same or not overlap).
+ *   includes room to run segments of them in parallel (V up to 256).  A
+ *   smaller workspace that holds the rest is accepted and runs every sequence
+ *   in order, and so does a call with final_state == initial_state (the state
+ *   updated in place; the two must be the same or not overlap).
  */
 int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                      int64_t HV);

@@ -233,9 +233,6 @@ def test_slow_heads_lose_no_precision(dev, beta_to, decay_to, mean):
 def test_offered_segments_are_taken(dev, N, HV, T, offered, kind):
     from torch_npu_ops_amd import _lib
     need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV), _least_workspace(T, N, HV)
-    assert (need > least + 256) == offered
-    if not offered:
-        return
     if kind == "equal":
         lens = [T // N] * N
     elif kind == "ragged":
@@ -246,7 +243,34 @@ def test_offered_segments_are_taken(dev, N, HV, T, offered, kind):
     q, k, v, g, beta, h0, cu = _inputs(lens, 1, HV, seed=T)
     t = [x.to(dev).contiguous() for x in (q, k, v, g, beta, cu)]
     h0 = h0.to(dev)
-    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
     _call(t, torch.empty_like(h0), h0, ws, need)
+    if not offered:
+        assert (ws[least:] == 0xA5).all()
+        return
     per = int(ws[least:least + 4].view(torch.int32))  # chunks per segment
     assert 0 < per < (max(lens) + 63) // 64
+
+
+@pytest.mark.parametrize("HV,V,T", [(8, 64, 4096), (8, 192, 4096), (4, 256, 4096), (16, 64, 8192),
+                                    (24, 64, 16384), (8, 320, 4096)])
+def test_every_width_fits_the_advertised_workspace(dev, HV, V, T):
+    """The size does not know V: with it, states of every width up to 256 take
+    their segments (wider ones run in order, with the in-order bits), and one
+    byte less runs in order."""
+    from torch_npu_ops_amd import _lib
+    q, k, v, g, beta, h0, cu = _inputs([T], 2, HV, seed=V, V=V)
+    t = [x.to(dev).contiguous() for x in (q, k, v, g, beta, cu)]
+    h0 = h0.to(dev)
+    need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, 1, HV), _least_workspace(T, 1, HV)
+    out = {}
+    for size in (need, need - 1, least):
+        ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+        fin = torch.empty_like(h0)
+        o = _call(t, fin, h0, ws, size, V=V)
+        segmented = bool(ws[least:least + 4].any())
+        assert segmented == (size == need and V <= 256)
+        out[size] = (o, fin, None)
+    assert torch.equal(out[need - 1][0], out[least][0])
+    assert torch.equal(out[need - 1][1], out[least][1])
+    _same(out[need], out[least])

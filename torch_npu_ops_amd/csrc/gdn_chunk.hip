@@ -1479,8 +1479,11 @@ SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t
   };
   // (At least 2 us must be gained: the model is good to a few percent.)
   float best = cost(1, longest, 0, N * tiles) - 2.f;
+  int64_t last = 0;
   for (int s = 2; s <= 64; ++s) {
     const int64_t len = cdiv(longest, s), segs = N * cdiv(longest, len);
+    if (len == last) continue;
+    last = len;
     const float c = cost(s, len, (segs - N) * (tiles + 2 * HV), segs * tiles);
     if (c < best) {
       best = c;
@@ -1502,6 +1505,9 @@ using namespace xk;
 
 namespace {
 
+// Widest states that the size makes room for; wider ones run in order.
+constexpr int64_t kSegMaxV = 256;
+
 // The least a call runs in (without segments).
 int64_t least_workspace(int64_t total_tokens, int64_t N, int64_t HV) {
   const int64_t nt = nt_max(total_tokens, N);
@@ -1513,9 +1519,11 @@ int64_t least_workspace(int64_t total_tokens, int64_t N, int64_t HV) {
 extern "C" int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                                 int64_t HV) {
   if (total_tokens < 0 || num_seqs < 0 || HV <= 0) return -1;
-  // Room for the segments of 128 x 128 states; wider ones run without.
-  return least_workspace(total_tokens, num_seqs, HV) +
-         seg_plan(total_tokens, num_seqs, HV, 128, 128).bytes;
+  // V is not known here: room for the segments of any up to kSegMaxV.
+  int64_t seg = 0;
+  for (int64_t V = 64; V <= kSegMaxV; V += 64)
+    seg = std::max(seg, seg_plan(total_tokens, num_seqs, HV, 128, V).bytes);
+  return least_workspace(total_tokens, num_seqs, HV) + seg;
 }
 
 namespace xk {
@@ -1615,8 +1623,9 @@ extern "C" int xk_gdn_chunk_fwd_strided(
                   s1 = reinterpret_cast<uintptr_t>(final_state);
   const uintptr_t state_bytes = static_cast<uintptr_t>(N * HV * K * V) * 4;
   const bool in_place = s0 && s1 && s0 < s1 + state_bytes && s1 < s0 + state_bytes;
-  const SegPlan plan = in_place ? SegPlan{} : seg_plan(total_tokens, N, HV, K, V);
-  if (plan.segs && static_cast<int64_t>(workspace_bytes) >= need + plan.bytes) {
+  const SegPlan plan = in_place || V > kSegMaxV ? SegPlan{} : seg_plan(total_tokens, N, HV, K, V);
+  if (plan.segs && static_cast<int64_t>(workspace_bytes) >=
+                       xk_gdn_chunk_workspace_bytes(total_tokens, N, HV)) {
     char* seg = p.rec + p.NTmax * HV * kRec;
     p.seg_max = plan.segs;
     p.seg_cus = num_cus();
