@@ -320,3 +320,15 @@ def test_v2_short_sequences(dev, lens, dim, W, layout, spec, dtype):
     live = torch.cat([torch.full((n,), bool(s != -1)) for n, s in zip(lens, slots)])
     torch.testing.assert_close(out.float().cpu()[live], ref[live], **_tol(dtype))
     assert torch.equal(st.cpu(), ref_state.to(dtype))
+
+
+# Around the lines between the two kernels: odd rows change over at 8 drafts
+# instead of 24 and take two channels a lane where that fills the chip; 4-byte
+# types take one (a block's states of 17 to 26 entries through its LDS).
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("layout", ["dense", "apart"])
+@pytest.mark.parametrize("lens,dim", [
+    ([8, 3], 1030), ([9, 2], 1030), ([2] * 128, 1030), ([2] * 64, 1030), ([16, 9], 1024),
+    ([24, 7], 768), ([25, 3], 768), ([8, 8], 257)])
+def test_v2_short_sequences_at_the_line(dev, lens, dim, layout, dtype):
+    test_v2_short_sequences(dev, lens, dim, 4, layout, True, dtype)

@@ -518,7 +518,7 @@ __global__ void __launch_bounds__(256) conv1d_varlen_kernel(VarlenParams p) {
 
 // ---------------------------------------------------------------------------
 // Varlen batches of short sequences (speculative verification, decode through
-// the varlen entry): one lane per (sequence, VEC channels), which loads the
+// the varlen entry): one lane per (sequence, 4 bytes of channels), which loads the
 // window, the state entries it keeps and the first tokens at once, walks its
 // tokens and writes the state.  The tile kernel has one lane per (16 tokens,
 // 2 to 4 channels): a few sequences' tokens fill a fraction of the CUs there,
@@ -535,7 +535,9 @@ __global__ void __launch_bounds__(256) conv1d_varlen_kernel(VarlenParams p) {
 // it alone.  32 sequences of 8 tokens take 7.1 us here and 11.5 in the tile
 // kernel, of 16 tokens 8.9 and 8.2; with speculative windows, whose states
 // grow with the draft, 32 of 16 take 11.5 and 28.7, 64 of 24 27.8 and 179,
-// 8 of 32 22.1 and 21.3.
+// 8 of 32 22.1 and 21.3.  In rows that the tile kernel reads one channel a
+// lane (odd widths or alignments) it has more lanes to walk: the line is 8
+// with windows too (256 of 16 drafts x 8,191 channels 167 here, 155 there).
 constexpr int64_t kShortLen = 8, kShortSpecLen = 24;
 constexpr int64_t kShortLds = 32768;  // most LDS for a block's states
 constexpr int kShortTok = 4;   // tokens loaded together
@@ -713,12 +715,23 @@ int launch_varlen(VarlenParams p, xk_dtype dt, hipStream_t s) {
   const bool vec = p.D % kV == 0 && p.sx % kV == 0 && p.so % kV == 0 &&
                    aligned(p.x, 16) && aligned(p.out, 16);
   p.w_vec = p.wdt == dt && p.swd == p.W && p.sww == 1 && aligned(p.w, 16);
-  const int64_t short_len = p.accepted ? kShortSpecLen : kShortLen;
+  const int64_t short_len = p.accepted && vec ? kShortSpecLen : kShortLen;
   if (p.max_query_len <= short_len && p.num_tokens <= short_len * p.B &&
       cdiv(p.D, 256) * p.B <= INT32_MAX) {
-    const bool pair = p.D % 2 == 0 && p.sx % 2 == 0 && p.so % 2 == 0 &&
-                      aligned(p.x, 2 * sizeof(T)) && aligned(p.out, 2 * sizeof(T));
-    return pair ? launch_short_w<T, 2>(p, s) : launch_short_w<T, 1>(p, s);
+    // Two channels of 2 bytes a lane, one of 4: two of those double the lane's
+    // chain, and a block's states no longer fit its LDS from 17 entries on (32
+    // sequences of 24 fp32 drafts x 8,192 channels 107.6 against 24.7 us).
+    // Odd rows take two where that still fills the chip (1 sequence of 8 x 130
+    // channels: 5.8 us with two, 4.8 with one, 4.9 in the tile kernel; 256 x
+    // 4,098: 19.8, 21.5 and 31.8) and no window's entries are moved one by one
+    // (their states are rarely aligned for the LDS: 256 windows of 8 x 4,098
+    // channels 48.0, 32.2 and 44.7).
+    if constexpr (sizeof(T) == 2) {
+      const bool pair = p.D % 2 == 0 && p.sx % 2 == 0 && p.so % 2 == 0 && aligned(p.x, 4) &&
+                        aligned(p.out, 4);
+      if (vec || (pair && !p.accepted && cdiv(p.D, 512) * p.B >= num_cus())) return launch_short_w<T, 2>(p, s);
+    }
+    return launch_short_w<T, 1>(p, s);
   }
   if (!vec) return launch_varlen_w<T, 1>(p, s);
   // 8 bytes of channels per lane, 4 where that makes at most two rounds of
