@@ -332,3 +332,27 @@ def test_v2_short_sequences(dev, lens, dim, W, layout, spec, dtype):
     ([24, 7], 768), ([25, 3], 768), ([8, 8], 257)])
 def test_v2_short_sequences_at_the_line(dev, lens, dim, layout, dtype):
     test_v2_short_sequences(dev, lens, dim, 4, layout, True, dtype)
+
+
+# Every width of a lane of the tile kernel: 2-byte types 4 and 8 bytes (16 for
+# output rows 32 KB apart), 4-byte types one, two and four channels, with
+# sequence edges inside tiles.
+@pytest.mark.parametrize("dtype,dim,tokens", [
+    (torch.bfloat16, 256, 100), (torch.bfloat16, 2048, 16000), (torch.bfloat16, 16384, 300),
+    (torch.float32, 256, 100), (torch.float32, 1024, 700), (torch.float32, 1024, 3000),
+    (torch.float32, 1024, 16500), (torch.float32, 8192, 300)])
+def test_v2_lane_widths(dev, dtype, dim, tokens):
+    from torch_npu_ops_amd import ops
+    g = torch.Generator().manual_seed(tokens + dim)
+    lens = [tokens // 3 - 5, 2, tokens - tokens // 3 - 30, 33]
+    x = _rn((tokens, dim), g, dtype)
+    w = _rn((dim, 4), g, dtype, 0.5)
+    state = _rn((6, dim, 3), g, dtype)
+    slots = torch.tensor([4, 0, 3, 1], dtype=torch.int32)
+    qsl = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    ref, ref_state = oc.causal_conv1d_update_v2(x, state, w, None, True, slots, qsl, max(lens))
+    st = state.to(dev)
+    out = ops.npu_causal_conv1d_update_v2(x.to(dev), st, w.to(dev), True, None, slots.to(dev),
+                                          qsl.to(dev), max(lens))
+    torch.testing.assert_close(out.float().cpu(), ref, **_tol(dtype))
+    assert torch.equal(st.cpu(), ref_state.to(dtype))

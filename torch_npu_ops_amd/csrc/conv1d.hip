@@ -734,17 +734,39 @@ int launch_varlen(VarlenParams p, xk_dtype dt, hipStream_t s) {
     return launch_short_w<T, 1>(p, s);
   }
   if (!vec) return launch_varlen_w<T, 1>(p, s);
-  // 8 bytes of channels per lane, 4 where that makes at most two rounds of
-  // resident waves (8 on a SIMD).  A lane of 16 bytes holds weights, window
-  // and a run of tokens in 141 registers, 3 waves on a SIMD; 8 bytes take 82
-  // (5 waves) and 4 fewer still: small calls have too few waves to hide the
-  // chain of lookups, window and tokens, large ones then run their accesses
-  // too narrow.  MI355X, us per call at 16 / 8 / 4 bytes: 4,096 tokens x
-  // 2,048 bf16 channels 16.8 / 12.6 / 10.5, 8,192 x 4,096 37.4 / 31.6 / 26.5,
-  // 8,192 x 8,192 54.2 / 51.5 / 62.0, 16,384 x 8,192 95.9 / 95.8 / 123.
-  const int64_t waves = cdiv(p.D, kWave * (kV / 4)) * cdiv(p.num_tokens, kTileT);
-  if (waves <= int64_t{2} * 8 * 4 * num_cus()) return launch_varlen_w<T, kV / 4>(p, s);
-  return launch_varlen_w<T, kV / 2>(p, s);
+  // Channels per lane.  MI355X, us per call, buffers rotated past the caches
+  // unless noted; "ragged" is 4 or 16 sequences.
+  //
+  // Output rows a multiple of 32 KB apart take 16 bytes a lane: narrower
+  // stores to the same channels of many such rows are slow (4,096 tokens at 16
+  // / 8 / 4 bytes: 16,384 bf16 channels 54 / 68 / 74, 8,192 fp32 ones 57 / 65 /
+  // 60; rows of 24 or 48 KB are not, nor inputs 32 KB apart).  Up to 256 tokens
+  // latency counts for more (14 / 10 / 9 at 64).
+  if (p.so * static_cast<int64_t>(sizeof(T)) % 32768 == 0 && p.num_tokens > 256)
+    return launch_varlen_w<T, kV>(p, s);
+  const int64_t tiles = cdiv(p.num_tokens, kTileT), cus = num_cus();
+  if constexpr (sizeof(T) == 2) {
+    // 8 bytes, 4 where that makes at most 1.5 rounds of resident waves (8 on a
+    // SIMD).  A lane of 16 bytes holds weights, window and a run of tokens in
+    // 141 registers, 3 waves on a SIMD; 8 bytes take 82 (5 waves) and 4 fewer
+    // still: small calls have too few waves to hide the chain of lookups,
+    // window and tokens, large ones then run their accesses too narrow.  At
+    // 16 / 8 / 4 bytes: 2,048 tokens x 4,096 channels 17 / 13 / 10, 6,144 x
+    // 4,096 30 / 27 / 24, 8,192 x 4,096 33 / 31 / 35 (in cache 30 / 29 / 26),
+    // 16,384 x 8,192 97 / 96 / 118.
+    if (cdiv(p.D, kWave * 2) * tiles <= 48 * cus) return launch_varlen_w<T, kV / 4>(p, s);
+    return launch_varlen_w<T, kV / 2>(p, s);
+  } else {
+    // Four channels of 4 bytes take the registers of 8 bytes above.  Fewer pay
+    // where there are next to no waves (one where four make at most half a
+    // wave per CU, two up to two waves) and, by a little, from 16 waves a CU
+    // on; in between ragged batches lose (2,048 x 4,096, 4 and 2 channels,
+    // ragged: 18.2 and 19.4; 256 x 8,192 16 and 12; 8,192 x 4,096 57 and 50).
+    const int64_t waves = cdiv(p.D, kWave * 4) * tiles;
+    if (2 * waves <= cus) return launch_varlen_w<T, kV / 4>(p, s);
+    if (waves <= 2 * cus || waves >= 16 * cus) return launch_varlen_w<T, kV / 2>(p, s);
+    return launch_varlen_w<T, kV>(p, s);
+  }
 }
 
 }  // namespace
