@@ -4,12 +4,12 @@ against the same call in a workspace one byte too small for the segments,
 which runs whole sequences in order.
 
 The two paths differ only in how the state reaches a segment: its entry state
-passes through the segments' transition matrices, whose products keep ~16
-mantissa bits like every state product of a chunk.  Each of the two paths is
-within 3.1e-5 (RMS + |value|) of the fp32 reference over the chunked tests
-(errors of 2^-17 of the state's size per product, over the few chunks for
-which the delta rule remembers them), so they may differ by twice that:
-6.2e-5 of the RMS and of the value.
+passes through the segments' transition matrices, to 24 bits, and what each
+segment adds is formed from a zero state.  Each of the two paths is within
+3.1e-5 (RMS + |value|) of the fp32 reference over the chunked tests (errors of
+2^-17 of the state's size per product, over the few chunks for which the delta
+rule remembers them), so they may differ by twice that: 6.2e-5 of the RMS and
+of the value.
 Outputs are sums of products of operands rounded to bf16 (the state's hi part,
 v_new); a difference that small can flip the last bit of one operand, which
 moves an output by up to 2^-8 of one term of its sum, a term being at most of
@@ -274,3 +274,114 @@ def test_every_width_fits_the_advertised_workspace(dev, HV, V, T):
     assert torch.equal(out[need - 1][0], out[least][0])
     assert torch.equal(out[need - 1][1], out[least][1])
     _same(out[need], out[least])
+
+
+def _segmented(dev, x, V=128):
+    """The call with and without segments: (o, final) of each, after checking
+    that each ran as meant."""
+    from torch_npu_ops_amd import _lib
+    q, k, v, g, beta, h0, cu = x
+    t = [a.to(dev).contiguous() for a in (q, k, v, g, beta, cu)]
+    h0 = h0.to(dev)
+    T, HV, N = q.shape[1], v.shape[2], cu.numel() - 1
+    need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV), _least_workspace(T, N, HV)
+    out = []
+    for size in (need, least):
+        ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+        fin = torch.empty_like(h0)
+        o = _call(t, fin, h0, ws, size, V=V)
+        assert bool(ws[least:least + 4].any()) == (size == need)
+        out.append((o, fin, None))
+    return out
+
+
+# Segments (checked to be there) of one to four 64-column tiles; empty and
+# one-token sequences beside segmented ones; odd lengths.
+@pytest.mark.parametrize("lens,H,HV,V", [
+    ([2500], 2, 6, 64), ([64 * 63 + 1, 0, 1, 1900], 2, 4, 128), ([3000, 200, 1500], 1, 1, 128),
+    ([5000, 1], 1, 2, 192), ([4097], 2, 4, 192), ([3333], 1, 2, 256)])
+def test_segments_and_order_agree(dev, lens, H, HV, V):
+    x = _inputs(lens, H, HV, seed=sum(lens) + V, V=V)
+    a, b = _segmented(dev, x, V)
+    _same(a, b)
+    q, k, v, g, beta, h0, cu = x
+    ro, rs = og.chunk_gdn(q, k, v, g, beta, None, h0, cu, use_qk_l2norm=True)
+    torch.testing.assert_close(a[0].float().cpu(), ro, **O_TOL)
+    assert_state_close(a[1].cpu(), rs)
+
+
+@pytest.mark.parametrize("opt", ["no_initial", "no_final", "bf16_g", "f32_beta", "i64_cu",
+                                 "wide_rows", "raw_keys"])
+def test_segments_with_other_arguments(dev, opt):
+    from torch_npu_ops_amd import _lib, ops
+    lens, H, HV = [2111, 1, 3000], 2, 4
+    q, k, v, g, beta, h0, cu = _inputs(lens, H, HV, seed=31)
+    if opt == "raw_keys":
+        q, k = F.normalize(q.float(), dim=-1).bfloat16(), F.normalize(k.float(), dim=-1).bfloat16()
+    T, N = q.shape[1], len(lens)
+    g = g.bfloat16() if opt == "bf16_g" else g
+    beta = beta.float() if opt == "f32_beta" else beta
+    cu = cu.long() if opt == "i64_cu" else cu
+    t = [a.to(dev).contiguous() for a in (q, k, v, g, beta, cu)]
+    sqk, sv = H * 128, HV * 128
+    if opt == "wide_rows":  # slices of one row, as the conv's output
+        row = torch.cat([a.reshape(T, -1) for a in t[:3]] + [t[0].new_zeros(T, 72)], 1)
+        t[0], t[1], t[2] = row, row[:, sqk:], row[:, 2 * sqk:]
+        sqk = sv = row.size(1)
+    h0d = None if opt == "no_initial" else h0.to(dev)
+    need, least = _lib.lib().xk_gdn_chunk_workspace_bytes(T, N, HV), _least_workspace(T, N, HV)
+    out = []
+    for size in (need, least):
+        ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+        o = torch.empty(1, T, HV, 128, dtype=torch.bfloat16, device=dev)
+        fin = None if opt == "no_final" else torch.empty(N, HV, 128, 128, device=dev)
+        st = _lib.lib().xk_gdn_chunk_fwd_strided(
+            t[0].data_ptr(), t[1].data_ptr(), sqk, t[2].data_ptr(), sv, _lib.XK_BF16,
+            t[3].data_ptr(), ops.xk_dtype(t[3]), t[4].data_ptr(), ops.xk_dtype(t[4]), o.data_ptr(),
+            ops._ptr(h0d), ops._ptr(fin), t[5].data_ptr(), ops.xk_dtype(t[5]), N, T, H, HV, 128, 128,
+            128 ** -0.5, int(opt != "raw_keys"), ws.data_ptr(), size, ops._stream(o))
+        _lib.check(st, "xk_gdn_chunk_fwd_strided")
+        assert bool(ws[least:least + 4].any()) == (size == need)
+        out.append((o, torch.zeros(1, device=dev) if fin is None else fin, None))
+    _same(*out)
+    ro, rs = og.chunk_gdn(q, k, v, g.float(), beta.float(), None, None if h0d is None else h0, cu,
+                          use_qk_l2norm=opt != "raw_keys")
+    torch.testing.assert_close(out[0][0].float().cpu(), ro, **O_TOL)
+    if opt != "no_final":
+        assert_state_close(out[0][1].cpu(), rs)
+
+
+def test_segments_through_the_cpp_api_on_views(dev):
+    """Slices of a wider row, long enough to be segmented, give bit for bit
+    what contiguous copies of them and the C call give."""
+    from torch_npu_ops_amd import _xk_torch as xt
+    q, k, v, g, beta, h0, cu = [x.to(dev) for x in _inputs([3000, 700], 2, 4, seed=41)]
+    T = q.shape[1]
+    row = torch.cat([a.reshape(T, -1) for a in (q, k, v)] + [q.new_zeros(T, 64)], 1)
+    parts = [p.view(1, T, -1, 128) for p in row[:, :1024].split([256, 256, 512], -1)]
+    out = [xt.npu_chunk_gated_delta_rule(*a, g, beta, initial_state=h0, output_final_state=True,
+                                         cu_seqlens=cu, use_qk_l2norm_in_kernel=True)
+           for a in (parts, (q, k, v))]
+    seg, _ = _segmented(dev, [x.cpu() for x in (q, k, v, g, beta, h0, cu)])
+    for o, fin in out:
+        assert torch.equal(o, seg[0]) and torch.equal(fin, seg[1])
+
+
+@pytest.mark.parametrize("T,HV", [(3000, 4), (26000, 8)])
+def test_segments_without_a_workspace_argument(dev, T, HV):
+    """The static buffer holds the segments of the first size (same bits as the
+    full workspace) and only the records of the second (bits of the order)."""
+    from torch_npu_ops_amd import _lib, ops
+    x = _inputs([T], 2, HV, seed=51)
+    want = _segmented(dev, x)
+    need = _lib.lib().xk_gdn_chunk_workspace_bytes(T, 1, HV)
+    q, k, v, g, beta, h0, cu = [a.to(dev).contiguous() for a in x]
+    o, fin = torch.empty_like(v), torch.empty_like(h0)
+    st = _lib.lib().xk_gdn_chunk_fwd_noalloc(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.XK_BF16, g.data_ptr(), _lib.XK_F32,
+        beta.data_ptr(), _lib.XK_BF16, o.data_ptr(), h0.data_ptr(), fin.data_ptr(), cu.data_ptr(),
+        _lib.XK_I32, 1, T, 2, HV, 128, 128, 128 ** -0.5, 1, ops._stream(o))
+    _lib.check(st, "xk_gdn_chunk_fwd_noalloc")
+    assert (need <= 64 << 20) == (T == 3000)
+    o2, fin2, _ = want[0 if need <= 64 << 20 else 1]
+    assert torch.equal(o, o2) and torch.equal(fin, fin2)
