@@ -266,3 +266,34 @@ def test_recurrent_token_counts(dev, K, V):
         ro, rs = og.recurrent_gdn(q, kk, v, g, beta, 0.1, h0, cu, idx, use_qk_l2norm=l2norm)
         torch.testing.assert_close(o[0].float().cpu(), ro.float(), **O_TOL)
         assert_state_close(s.cpu(), rs)
+
+
+@pytest.mark.parametrize("size", [0.0, 1e-6, 1e-3, 1.0, 1e15, 1e20])
+def test_key_norms_from_nothing_to_overflow(dev, size):
+    """Raw keys of every size: 1 / sqrt(sum k^2 + 1e-6) from 1e3 (zero keys)
+    down to 0 where the sum overflows (the key then vanishes).  fp32
+    throughout: sums of 128 products, a few roundings of each factor."""
+    from torch_npu_ops_amd import ops
+    gen = torch.Generator().manual_seed(9)
+    T, H, HV = 5, 1, 2
+    q = torch.randn(1, T, H, 128, generator=gen)
+    k = torch.randn(1, T, H, 128, generator=gen) * size
+    v = torch.randn(1, T, HV, 128, generator=gen)
+    g = -torch.rand(1, T, HV, generator=gen)
+    beta = torch.rand(1, T, HV, generator=gen)
+    h0 = torch.randn(1, HV, 128, 128, generator=gen)
+    o, fin = ops.npu_fused_recurrent_gated_delta_rule(
+        *(x.to(dev) for x in (q, k, v, g, beta)), initial_state=h0.to(dev),
+        inplace_final_state=False,
+        cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=dev))
+    s, want = h0[0].double(), []
+    for t in range(T):
+        qn, kn = (x[0, t, 0].double() for x in (q, k))
+        qn = qn / (qn.pow(2).sum() + 1e-6).sqrt() * 128 ** -0.5
+        kn = kn * 0 if size == 1e20 else kn / (kn.pow(2).sum() + 1e-6).sqrt()
+        s = s * g[0, t].double().exp()[:, None, None]
+        new = beta[0, t].double()[:, None] * (v[0, t].double() - (s * kn[:, None]).sum(-2))
+        s = s + kn[:, None] * new[:, None, :]
+        want.append((s * qn[:, None]).sum(-2))
+    torch.testing.assert_close(fin[0].cpu().double(), s, rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(o[0].cpu().double(), torch.stack(want), rtol=1e-5, atol=1e-5)
