@@ -350,7 +350,7 @@ int xk_gdn_conv_gating_decode(
  *   (triton_npu/torch_api/triton_ops_api.h:111-122,
  *    npu_triton_chunk_gated_delta_rule.cpp:556-642) -- the whole pipeline
  * of cumsum, scaled K K^T, solve_tril, WY recompute, state recurrence and
- * output (a6b-a6g) in three launches with no host synchronisation.
+ * output (a6b-a6g) in two to four launches with no host synchronisation.
  *   q, k : [total_tokens, H, K]; v, o : [total_tokens, HV, V] (dtype
  *   bf16, as the reference requires); g : [total_tokens, HV] log-decay,
  *   beta : [total_tokens, HV] (each fp32 or bf16); sequences
@@ -365,7 +365,13 @@ int xk_gdn_conv_gating_decode(
  *   includes room to run segments of them in parallel (V up to 256).  A
  *   smaller workspace that holds the rest is accepted and runs every sequence
  *   in order, and so does a call with final_state == initial_state (the state
- *   updated in place; the two must be the same or not overlap).
+ *   updated in place; the two must be the same or not overlap).  The two forms
+ *   agree to the tolerance of the state's arithmetic, not bit for bit; which
+ *   one a sequence takes, and its segments, follow from the whole batch.
+ *   The size is for the current device (its compute units) and for exactly
+ *   this (total_tokens, num_seqs, HV): a smaller batch can ask for more than a
+ *   larger one.  A buffer sized once for the most tokens and sequences is
+ *   always enough to run in, but may run some smaller calls in order.
  */
 int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t num_seqs,
                                      int64_t HV);
@@ -394,10 +400,12 @@ int xk_gdn_chunk_fwd_strided(
  * xk_gdn_chunk_fwd without a workspace argument, for callers that cannot
  * allocate device memory (code under hipGraph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.
- * Same arguments and results as xk_gdn_chunk_fwd (the same kernels run);
- * the workspace is a static device buffer of 64 MiB that the library holds
- * on every GPU it runs on until the process ends.  Calls whose workspace
- * without room for segments exceeds 64 MiB return XK_ERR_SCRATCH (e.g. up to ~6,700 tokens at HV = 32, ~27,000 at HV = 8).
+ * Same arguments and results as xk_gdn_chunk_fwd in a workspace of 64 MiB:
+ * the workspace is a static device buffer of that size that the library holds
+ * on every GPU it runs on until the process ends.  A call whose segments do
+ * not fit it runs every sequence in order.  Calls whose workspace without
+ * room for segments exceeds 64 MiB return XK_ERR_SCRATCH (they fit up to
+ * ~6,700 tokens at HV = 32, ~27,000 at HV = 8).
  * The call allocates nothing; `stream` must belong to the current device.
  * Every call on one GPU shares that GPU's buffer: calls that overlap in
  * time on one GPU (other streams, other host threads) race.

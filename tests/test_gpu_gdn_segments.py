@@ -74,7 +74,7 @@ def _same(a, b):
 
 # One sequence at its shortest segmented length, odd lengths around chunk and
 # segment edges, many segments; ragged batches with empty and one-token
-# sequences; one and three 64-column tiles.
+# sequences; one and two 64-column tiles.
 @pytest.mark.parametrize("lens,H,HV,V", [
     ([1024], 4, 8, 128), ([1025], 2, 4, 128), ([2111], 1, 2, 128), ([4095], 2, 2, 128),
     ([9000], 1, 2, 128), ([2500], 2, 6, 64), ([64 * 31 + 1, 0, 1, 700], 2, 4, 128),

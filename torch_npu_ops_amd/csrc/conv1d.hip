@@ -26,8 +26,8 @@
 // shift = len.  A "prefill" rule (state_len_run = eff_state_len for every
 // sequence, i.e. the last W-1 inputs) is offered for full-prefill callers.
 //
-// Design: channels are the vector dimension (16-byte accesses along the
-// contiguous channel axis); each lane walks a tile of tokens with the W-1
+// Design: channels are the vector dimension (accesses of 4 to 16 bytes along
+// the contiguous channel axis); each lane walks a tile of tokens with the W-1
 // previous inputs in a register window, so every x element is read from
 // HBM once (plus a W-1 token halo per tile, served from L2) and every output
 // written once.  Sequence boundaries inside a tile restart the window from

@@ -16,7 +16,8 @@
 // (npu_l2norm_last_dim, x / sqrt(sum x^2 + 1e-6)) is folded in as per-token
 // row scales, so the matrix products always see the exact bf16 inputs.
 //
-// Two to five launches, no host synchronisation (capturable in a hipGraph):
+// Two launches (three above 64 sequences, four with segments), no host
+// synchronisation (capturable in a hipGraph):
 //  * P0 (one small block, above 64 sequences) turns cu_seqlens into chunk
 //    offsets.
 //  * P1, fully parallel, one wave per (chunk, v-head), computes everything
@@ -24,9 +25,9 @@
 //    (chunk, head) to the workspace:
 //      - Ai = (I + M)^-1 as a bf16 hi/lo pair (hi + lo carries ~16 mantissa
 //        bits).  K K^T runs on bf16 MFMA (exact products, fp32 sums); the
-//        inverse inverts the two 32x32 diagonal blocks by forward
-//        substitution (one lane per column) and forms the off-diagonal block
-//        X10 = -X11 M10 X00 with hi/lo-split MFMAs;
+//        inverse inverts the four 16x16 diagonal blocks by forward
+//        substitution (one lane per column) and merges them, X10 = -X11 M10
+//        X00, with hi/lo-split MFMAs (invert_unit_lower);
 //      - Aq = scale * tril(r_q r_k (q k^T) exp(gc_i - gc_j)) in bf16 (it only
 //        feeds the bf16 output);
 //      - per-token factors cq = scale exp(gc) r_q, ck = b exp(gc) r_k, b,
@@ -166,7 +167,10 @@ constexpr int64_t kSegSeqs = 16;            // most sequences (the plan loops ov
 // one engine, so the places that idle blocks leave are not taken by others
 // (3 segments x 24 heads, 240 blocks of 288 with work, take two rounds of 256
 // CUs).  A step takes 1.6 (sum) or 2.35 us (out) on an idle chip and about
-// 0.6 us more on a full one, a step of the combine kernel 1.4 us.
+// 0.6 us more on a full one, a step of the combine kernel 1.4 us.  Against
+// traced passes (MI355X, one sequence of 8 v-heads) the sum of the three is
+// 69 (model) and 66 us at 4,096 tokens (8 segments), 277 and 260 at 32,768
+// (16).
 __host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, int cus) {
   auto time = [&](int blocks, float step) {
     const float load = static_cast<float>(blocks) / cus;
@@ -361,7 +365,7 @@ __global__ void __launch_bounds__(kTh) gdn_chunk_prep_kernel(ChunkParams p) {
   // An element then takes two multiplies instead of an exponential and six
   // VALU instructions.  c_k = r_k exp(G_{nj+1} - gc) is formed once per token.
   // 24 of an M or Aq tile's 40 elements per lane; the kernel at 16,384 tokens
-  // x 32 v-heads on MI355X: 80.5 -> 78.2 us.
+  // x 32 v-heads traced on one MI355X: 80.2 -> 78.2 us.
   ckv[lane] = rkv[lane] * __expf(gcv[lane | 15] - gv);
   float tile_decay[3];  // exp(G_mi - G_{nj+1}) of (2, 0), (3, 1), (3, 0)
   {
