@@ -1472,9 +1472,8 @@ struct SegPlan {
   int segs = 0;  // most segments; 0: whole sequences
   int64_t bytes = kSegHead;
 };
-SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t V) {
+SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t V, int cus) {
   SegPlan r;
-  const int cus = num_cus();
   const int64_t tiles = HV * (V / 64);
   if (N <= 0 || N > kSegSeqs || V % 64 != 0 || N * tiles > cus) return r;
   const int64_t longest = std::max<int64_t>(cdiv(cdiv(total_tokens, N), kC), 1);
@@ -1483,16 +1482,18 @@ SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t
   };
   // (At least 2 us must be gained: the model is good to a few percent.)
   float best = cost(1, longest, 0, N * tiles) - 2.f;
-  int64_t last = 0;
-  for (int s = 2; s <= 64; ++s) {
+  // The smallest s of every length, while s segments of one chunk could gain:
+  // every call pays for this loop (63 candidates per width took 0.3 us).
+  for (int64_t s = 2; s <= 64 && 25.f + 1.4f * (s - 2) < best;) {
     const int64_t len = cdiv(longest, s), segs = N * cdiv(longest, len);
-    if (len == last) continue;
-    last = len;
-    const float c = cost(s, len, (segs - N) * (tiles + 2 * HV), segs * tiles);
+    const float c =
+        cost(static_cast<int>(s), len, (segs - N) * (tiles + 2 * HV), segs * tiles);
     if (c < best) {
       best = c;
       r.segs = static_cast<int>(segs);
     }
+    if (len <= 1) break;
+    s = cdiv(longest, len - 1);
   }
   // Several sequences: room for one round of kSegOut blocks.
   if (r.segs && N > 1) r.segs = static_cast<int>(std::max<int64_t>(r.segs, cus / tiles) + N / 2);
@@ -1525,8 +1526,9 @@ extern "C" int64_t xk_gdn_chunk_workspace_bytes(int64_t total_tokens, int64_t nu
   if (total_tokens < 0 || num_seqs < 0 || HV <= 0) return -1;
   // V is not known here: room for the segments of any up to kSegMaxV.
   int64_t seg = 0;
+  const int cus = num_cus();
   for (int64_t V = 64; V <= kSegMaxV; V += 64)
-    seg = std::max(seg, seg_plan(total_tokens, num_seqs, HV, 128, V).bytes);
+    seg = std::max(seg, seg_plan(total_tokens, num_seqs, HV, 128, V, cus).bytes);
   return least_workspace(total_tokens, num_seqs, HV) + seg;
 }
 
@@ -1627,7 +1629,9 @@ extern "C" int xk_gdn_chunk_fwd_strided(
                   s1 = reinterpret_cast<uintptr_t>(final_state);
   const uintptr_t state_bytes = static_cast<uintptr_t>(N * HV * K * V) * 4;
   const bool in_place = s0 && s1 && s0 < s1 + state_bytes && s1 < s0 + state_bytes;
-  const SegPlan plan = in_place || V > kSegMaxV ? SegPlan{} : seg_plan(total_tokens, N, HV, K, V);
+  const SegPlan plan = in_place || V > kSegMaxV
+                           ? SegPlan{}
+                           : seg_plan(total_tokens, N, HV, K, V, num_cus());
   if (plan.segs && static_cast<int64_t>(workspace_bytes) >=
                        xk_gdn_chunk_workspace_bytes(total_tokens, N, HV)) {
     char* seg = p.rec + p.NTmax * HV * kRec;
