@@ -167,17 +167,20 @@ constexpr int64_t kSegSeqs = 16;            // most sequences (the plan loops ov
 // one engine, so the places that idle blocks leave are not taken by others
 // (3 segments x 24 heads, 240 blocks of 288 with work, take two rounds of 256
 // CUs).  A step takes 1.6 (sum) or 2.35 us (out) on an idle chip and about
-// 0.6 us more on a full one, a step of the combine kernel 1.4 us.  Against
+// 0.6 us more on one full of blocks with work (`work` of the sums; idle ones
+// counted there kept 2 sequences of 8,689 tokens x 32 v-heads whole, 432 us
+// against 411), a step of the combine kernel 1.4 us.  Against
 // traced passes (MI355X, one sequence of 8 v-heads) the sum of the three is
-// 69 (model) and 66 us at 4,096 tokens (8 segments), 277 and 260 at 32,768
+// 68 (model) and 66 us at 4,096 tokens (8 segments), 277 and 260 at 32,768
 // (16).
-__host__ __device__ inline float seg_cost(int s, int len, int sums, int outs, int cus) {
-  auto time = [&](int blocks, float step) {
-    const float load = static_cast<float>(blocks) / cus;
-    return fmaxf(1.f, ceilf(load)) * len * (step + 0.6f * fminf(1.f, load));
+__host__ __device__ inline float seg_cost(int s, int len, int sums, int work, int outs,
+                                          int cus) {
+  auto time = [&](int blocks, int busy, float step) {
+    const float load = static_cast<float>(busy) / cus;
+    return fmaxf(1.f, ceilf(static_cast<float>(blocks) / cus)) * len * (step + 0.6f * fminf(1.f, load));
   };
-  const float out = 8.f + time(outs, 2.35f);
-  return s <= 1 ? out : out + 14.f + time(sums, 1.6f) + 1.4f * (s - 2);
+  const float out = 8.f + time(outs, outs, 2.35f);
+  return s <= 1 ? out : out + 14.f + time(sums, work, 1.6f) + 1.4f * (s - 2);
 }
 
 // Chunks per segment for this batch, 0 for whole sequences (wave-uniform; N <=
@@ -189,10 +192,14 @@ __device__ __forceinline__ int wave_seg_len(const ChunkParams& p) {
   int longest = 1;
   for (int n = 0; n < N; ++n) longest = max(longest, __builtin_amdgcn_readlane(w.cnt, n));
   const int len = (longest + lane) / (lane + 1);
-  int segs = 0;
-  for (int n = 0; n < N; ++n)
-    segs += max((__builtin_amdgcn_readlane(w.cnt, n) + len - 1) / len, 1);
-  const float cost = seg_cost(lane + 1, len, (segs - N) * (p.seg_nvt + 2) * p.HV,
+  int segs = 0, cut = 0;  // cut: sequences of several segments
+  for (int n = 0; n < N; ++n) {
+    const int c = (__builtin_amdgcn_readlane(w.cnt, n) + len - 1) / len;
+    segs += max(c, 1);
+    cut += c > 1;
+  }
+  const int sums = (segs - N) * (p.seg_nvt + 2) * p.HV;
+  const float cost = seg_cost(lane + 1, len, sums, sums - cut * 2 * p.HV,
                               segs * p.seg_nvt * p.HV, p.seg_cus);
   // Smallest cost, the fewest segments among equals.
   int key = lane == 0 || segs <= p.seg_max ? static_cast<int>(fminf(cost * 16.f, 3e7f)) : 30000000;
@@ -1478,7 +1485,8 @@ SegPlan seg_plan(int64_t total_tokens, int64_t N, int64_t HV, int64_t K, int64_t
   if (N <= 0 || N > kSegSeqs || V % 64 != 0 || N * tiles > cus) return r;
   const int64_t longest = std::max<int64_t>(cdiv(cdiv(total_tokens, N), kC), 1);
   auto cost = [&](int s, int64_t len, int64_t sums, int64_t outs) {
-    return seg_cost(s, static_cast<int>(len), static_cast<int>(sums), static_cast<int>(outs), cus);
+    return seg_cost(s, static_cast<int>(len), static_cast<int>(sums),
+                    static_cast<int>(sums - N * 2 * HV), static_cast<int>(outs), cus);
   };
   // (At least 2 us must be gained: the model is good to a few percent.)
   float best = cost(1, longest, 0, N * tiles) - 2.f;
